@@ -26,14 +26,13 @@ unsigned long long next_launch_tag() {
   static const unsigned long long seed =
       (unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9E3779B97F4A7C15ull ^
       ((unsigned long long)getpid() << 32);
-  for (;;) {
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (seq.fetch_add(1) + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    z &= (1ull << 40) - 1;
-    if (z != 0) return z;
-  }
+  unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (seq.fetch_add(1) + 1);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  // 40 bits, the top one set: as a number a counter word with this tag is
+  // above a cleared word and above most stale bytes (open_counter)
+  return (z & ((1ull << 40) - 1)) | (1ull << 39);
 }
 
 // Compute units of the current device (cached per device id).
