@@ -177,6 +177,7 @@ struct DecodeArgs {
   int ghost;            // stream tokens charged per row for its fixed costs (multiple of 32)
   int slot_classes;     // residency slots per CU the grid fills (slice weighting classes)
   int slot_skew;        // slice weight skew between the first and last slot, in 1/1000
+  int slice_rows;       // rows the least slice length is reckoned for (min_slice); 0: a tile
   float qscale;         // softmax scale * log2(e) * 1/sqrt(D) (rotation norm)
   _Float16* out;
   float* ws_ml;         // [Hkv][slots][G][2]  (max, sum) of each segment
@@ -242,7 +243,22 @@ struct SliceLayout {
   int sz;       // lane c: slice length of class c
   int start;    // lane c: stream position of class c's first slice
 };
-__device__ __forceinline__ SliceLayout slice_layout(int total, int W, int ncls, int skew_permille, int lane) {
+// Least slice length of a stream of `total` tokens in `rows` rows.  Cutting a
+// row into S segments leaves each workgroup total / S of its tokens to stream
+// (about 0.013 us a token) but adds S arrivals at one counter word and S
+// partials for one workgroup to combine (about 0.2 us a segment), so the
+// time is least at slices of sqrt(15 x the mean row).  Measured against one
+// slice per resident workgroup (us a launch at head_dim 128): one row of
+// 30,011 tokens, 8 KV heads: 96 slices 36.4, 48 slices (629 tokens) 28.9, 32
+// slices 29.6; one K8V3 row of 20,000, 2 KV heads, group 8: 384 slices 92, 32
+// 27.5; 4 rows of about 2,000: 96 slices 19.6, 48 (183 tokens) 17.1.  Batches
+// that fill the GPU have longer slices anyway.
+constexpr float kSliceTokens = 15.0f;
+__device__ __forceinline__ int min_slice(int total, int rows) {
+  if (rows == 0) return kTile;
+  return padded32((int)__builtin_amdgcn_sqrtf(kSliceTokens * (float)total / (float)rows));
+}
+__device__ __forceinline__ SliceLayout slice_layout(int total, int W, int ncls, int skew_permille, int rows, int lane) {
   const int classes = max(1, min(ncls, min(W, kMaxResidentPerCU)));
   const bool act = lane < classes;
   SliceLayout s;
@@ -255,7 +271,7 @@ __device__ __forceinline__ SliceLayout slice_layout(int total, int W, int ncls, 
   ws += swz_xor_f<4>(ws);
   const float wsum = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ws), 0));
   const float unit = (float)total / wsum;
-  s.sz = act ? max(kTile, padded32((int)ceilf(unit * wt))) : 0;
+  s.sz = act ? max(max(kTile, min_slice(total, rows)), padded32((int)ceilf(unit * wt))) : 0;
   const int span = (s.f1 - s.f0) * s.sz;
   int incl = span;  // inclusive scan over lanes 0..7 (DPP row_shr: lanes below `off` read 0)
   incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, false);
@@ -360,7 +376,7 @@ struct SliceLoc {
 // Plan layout (int32 words): a header naming the launch geometry the plan was
 // made for, then one entry per workgroup column j.
 constexpr int kPlanHeader = 32;       // words before the entries (entries stay 64-byte aligned)
-constexpr int kPlanHeaderWords = 17;  // header words in use
+constexpr int kPlanHeaderWords = 18;  // header words in use
 constexpr int kPlanEntry = 16;
 constexpr int kPlanMagic = 0x50384B53;
 constexpr int kPlanAdaptWord = 16;  // header word: 1 when the slice bounds come from the adaptive area
@@ -406,6 +422,7 @@ __host__ __device__ inline int32_t plan_header_word(const DecodeArgs& a, int i) 
     case 12: return (int32_t)(uint32_t)(uintptr_t)a.context_lens;
     case 13: return (int32_t)(uint32_t)((uint64_t)(uintptr_t)a.context_lens >> 32);
     case 14: return (int32_t)a.bt_stride;
+    case 17: return a.slice_rows;
     default: return 0;
   }
 }
@@ -442,7 +459,7 @@ template <bool WIN>
 __device__ __forceinline__ bool locate_slice(const DecodeArgs& a, const int* lens_lds, int j, int lane, SliceLoc& s) {
   s.total = stream_total<WIN>(a, lens_lds, lane);
   s.L = 0;
-  const SliceLayout sl = slice_layout(s.total, a.wg_per_head, a.slot_classes, a.slot_skew, lane);
+  const SliceLayout sl = slice_layout(s.total, a.wg_per_head, a.slot_classes, a.slot_skew, a.slice_rows, lane);
   s.lo = slice_start(sl, j);
   if (s.lo >= s.total) return false;
   s.hi = j + 1 >= a.wg_per_head ? s.total : min(s.total, slice_start(sl, j + 1));
@@ -1460,7 +1477,7 @@ __global__ __launch_bounds__(64 * kDecWaves, D >= 256 ? 2 : 3) void decode_kerne
         } else {
           const SliceLayout sm = slice_layout(opaque_int(total), opaque_int(a.wg_per_head),
                                               opaque_int(a.slot_classes), opaque_int(a.slot_skew),
-                                              opaque_int(threadIdx.x) & 63);
+                                              opaque_int(a.slice_rows), opaque_int(threadIdx.x) & 63);
           jf = slice_of(sm, rs);
           jl = slice_of(sm, rs + padL - 1);
         }
@@ -1726,7 +1743,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void decode_bounds_kernel(DecodeArg
       run = __shfl(v, 63, 64);
     }
   } else {
-    const SliceLayout sl = slice_layout(total, W, a.slot_classes, a.slot_skew, lane);
+    const SliceLayout sl = slice_layout(total, W, a.slot_classes, a.slot_skew, a.slice_rows, lane);
     for (int c0 = 1; c0 < W; c0 += 64) {
       const int jj = c0 + lane;
       if (jj < W) bd[jj] = min(total, slice_start_lane(sl, jj));
@@ -1922,6 +1939,7 @@ static int launch_decode_impl(DecodeArgs& a, hipStream_t stream) {
     const int v = atoi(env);
     a.slot_classes = v < 1 ? 1 : (v > kMaxResidentPerCU ? kMaxResidentPerCU : v);
   }
+  a.slice_rows = getenv("S8KV_DECODE_WG_PER_HEAD") ? 0 : a.batch;  // (a forced grid keeps every slice it asks for)
   a.slot_skew = kSlotSkewPermille;
   if (const char* env = getenv("S8KV_DECODE_SLOT_SKEW")) a.slot_skew = atoi(env);
   if (const char* env = getenv("S8KV_DECODE_GHOST")) {
