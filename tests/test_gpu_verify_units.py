@@ -1,0 +1,82 @@
+"""The verify kernels' units on the GPU against the oracle: every (sequence, KV
+head, query block, key split) is computed by exactly one workgroup whatever the
+number of pairs (dispatch takes them gcd(pairs, 8) at a time), and equal key
+splits of rows of different lengths combine to the whole row's result."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import kv_oracle as O
+from superl8_serve_amd import _lib, ops
+from tests.kvcase import make_case
+from tests.kvgpu import CODEBOOK, alloc, append, assert_close, layer, t, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(seed, kind, hq, hkv, d, bs, prefix, nq, what, query_lens=None, window=None):
+    prefix = np.asarray(prefix)
+    case = make_case(seed, len(prefix), hq, hkv, d, bs, prefix + nq, outlier_channels=2 if d >= 128 else 0)
+    cache = alloc(kind, case.num_blocks, hkv, bs, d)
+    append(kind, t(case.k), t(case.v), cache, t(case.slots))
+    qv = np.random.default_rng(seed + 1).standard_normal((len(prefix), hq, nq, d)).astype(np.float16)
+    fn = ops.attn_paged_verify if kind == "int8" else ops.attn_paged_verify_k8v3
+    extra = () if kind == "int8" else (t(CODEBOOK),)
+    out = fn(t(qv), *cache, *extra, t(case.block_table), t(prefix.astype(np.int32)), bs,
+             query_lens=None if query_lens is None else t(np.asarray(query_lens, np.int32)),
+             max_context_len=int(case.lens.max()), scale=case.scale, window=window)
+    torch.cuda.synchronize()
+    ref = O.paged_verify(qv, layer(kind, tuple(to_np(x) for x in cache)), case.block_table, prefix, case.scale,
+                         query_lens=query_lens, window=window)
+    got = to_np(out.float())
+    for b, n in enumerate([] if query_lens is None else query_lens):
+        assert not got[b, :, n:].any(), f"{what}: row {b}, outputs past its {n} queries"
+    assert_close(got, ref, what)
+
+
+@pytest.mark.parametrize("batch,hkv", [(1, 1), (1, 4), (3, 1), (3, 2), (3, 4), (5, 3), (2, 8)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_every_unit_of_any_pair_count(batch, hkv, d):
+    """Several query blocks of 1, 3, 4, 6, 12, 15 and 16 pairs."""
+    nq = 70
+    _check(40 + batch * 8 + hkv, "int8", 4 * hkv, hkv, d, 16, [90 + 37 * b for b in range(batch)], nq,
+           f"{batch} x {hkv} pairs, D={d}")
+
+
+@pytest.mark.parametrize("batch,hkv", [(1, 2), (7, 1)])
+def test_dense_units_of_any_pair_count(batch, hkv):
+    rng = np.random.default_rng(60 + batch)
+    lens = [400 - 53 * b for b in range(batch)]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    hq, d = 4 * hkv, 128
+    q, k, v = (rng.standard_normal((cu[-1], h, d)).astype(np.float16) for h in (hq, hkv, hkv))
+    out = to_np(ops.attn_varlen(t(q), t(k), t(v), t(cu), t(cu), max(lens), max(lens), causal=True,
+                                scale=d ** -0.5).float())
+    for b, n in enumerate(lens):
+        qb, kb, vb = (torch.from_numpy(x[cu[b]:cu[b + 1]]).double().transpose(0, 1) for x in (q, k, v))
+        kb, vb = kb.repeat_interleave(4, 0), vb.repeat_interleave(4, 0)
+        s = (qb @ kb.transpose(1, 2)) * d ** -0.5
+        s = s.masked_fill(~torch.ones((n, n), dtype=torch.bool).tril(), float("-inf"))
+        assert_close(out[cu[b]:cu[b + 1]], (torch.softmax(s, -1) @ vb).transpose(0, 1).numpy(), f"sequence {b}")
+
+
+@pytest.mark.parametrize("kind,d", [("int8", 128), ("int8", 64), ("int8", 256), ("k8v3", 128), ("k8v3", 256)])
+@pytest.mark.parametrize("window", [None, 700])
+def test_equal_splits_of_ragged_rows(kind, d, window):
+    """The planned split of a batch of short and long rows with few queries:
+    rows ending at, one below and one past a split's last key and tile, an
+    empty prefix, and rows whose queries are fewer than the call's."""
+    prefix, nq = [2600, 0, 511, 512, 513, 1023, 1024, 31, 33], 5
+    lens = [5, 5, 1, 5, 0, 2, 5, 5, 3]
+    _check(80 + d, kind, 8, 2, d, 32, prefix, nq, f"{kind} D={d} window={window}", query_lens=lens, window=window)
+
+
+def test_workspace_counts_the_split():
+    """The workspace query plans the ragged batch's split too, and a call
+    without a workspace runs unsplit."""
+    lib = _lib.load()
+    assert lib.s8kv_verify_workspace_size(32, 32, 8, 128, 5, 8192) > 0
+    assert lib.s8kv_verify_workspace_size(32, 32, 8, 128, 5, 500) == 0
