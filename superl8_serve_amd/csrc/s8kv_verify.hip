@@ -105,10 +105,14 @@ struct VerifyArgs {
   int max_context_len;
   int n_qblocks;              // query blocks (rows_per_wg rows each) per (sequence, KV head)
   // split of the key range: workgroup split sp of a (sequence, KV head, query
-  // block) attends its share of the keys and writes unnormalized partials
-  // (acc[D], m_ref, l per row, pitch D + 4 floats) to part; a second kernel
-  // combines them.  splits == 1: the workgroup writes the output itself.
+  // block) attends keys split_keys * sp .. of the block's range (a short row
+  // has fewer non-empty splits) and writes unnormalized partials (acc[D],
+  // m_ref, l per row, pitch D + 4 floats, part_rows rows per unit) of its live
+  // 16- or 32-row groups to part; a second kernel combines them.  splits == 1:
+  // the workgroup writes the output itself.
   int splits;
+  int split_keys;             // multiple of kTile; split_keys * splits covers every block's range
+  int part_rows;
   float* part;
   int window;                 // verify_kernel<.., WIN>: only the last `window` prefix keys are visible
   // WIN, optional: the drafts' fresh K (rotated, fp32) and V (fp16),
@@ -148,6 +152,13 @@ __device__ __forceinline__ Unit unit_of(const VerifyArgs& a, int id) {
   const int u = rem / g;
   const int sp = u / a.n_qblocks;
   return {pg * g + (rem & (g - 1)), u - sp * a.n_qblocks, sp};
+}
+
+// Split sp of a block whose keys are [lo, end) (lo tile-aligned): [k_lo, k_hi).
+__device__ __forceinline__ void split_range(const VerifyArgs& a, int sp, int end, int& k_lo, int& k_hi) {
+  if (a.splits == 1) return;
+  k_lo += sp * a.split_keys;
+  if (sp + 1 < a.splits) k_hi = min(end, k_lo + a.split_keys);
 }
 
 // Position of tile key tt (0..31) in the LDS V tile: lane group g's eight
@@ -206,6 +217,10 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
   // position's bound on are visible to every row)
   const int lo_key = WIN ? max(0, prefix + (DENSE ? row0 / G : 0) - a.window) : 0;
   const int lo_all = WIN && DENSE ? prefix + min(nq - 1, (row0 + C::ROWS - 1) / G) - a.window : lo_key;
+  // this workgroup's keys: split sp of the block's tile-aligned key range
+  int k_lo = lo_key & ~(kTile - 1), k_hi = kv_end;
+  split_range(a, sp, kv_end, k_lo, k_hi);
+  if (a.splits > 1 && k_lo >= k_hi) return;  // no partial (the combine counts the splits with keys)
   // keys below vis_all are visible to every row of the block: the prefix, and
   // for a chain / causal block also the drafts up to its first position
   const int vis_all = tree ? prefix : prefix + row0 / G + 1;
@@ -302,13 +317,6 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
   const uint32_t hkv = (uint32_t)a.num_kv_heads;
   const int32_t* bt_row = a.block_table + (int64_t)b * a.bt_stride;
 
-  // this workgroup's keys: split sp of the block's tile-aligned key range
-  int k_lo = lo_key & ~(kTile - 1), k_hi = kv_end;
-  if (a.splits > 1) {
-    const int chunk = ((max(0, kv_end - k_lo) + a.splits - 1) / a.splits + kTile - 1) & ~(kTile - 1);
-    k_lo += sp * chunk;
-    k_hi = min(kv_end, k_lo + chunk);
-  }
   for (int u0 = k_lo; u0 < k_hi; u0 += kSubKeys) {
     const int u1 = min(k_hi, u0 + kSubKeys);
     const int fb = u0 >> bs_log2;
@@ -778,7 +786,8 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
     for (int rg = 0; rg < RG; ++rg) {
       const float l_tot = sum_x32(sum_x16(l_run[rg]));
       const int rl = (rg * C::WAVES + wave) * 16 + c;  // row within the block
-      float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * C::ROWS + rl) * (D + 4);
+      if ((row0 + rl - c) / G >= nq) continue;         // (no row of the group is read back)
+      float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * a.part_rows + rl) * (D + 4);
 #pragma unroll
       for (int n = 0; n < C::NPV; ++n) *reinterpret_cast<float4_t*>(pr + 16 * n + 4 * g) = acc[rg][n];
       if (g == 0) {
@@ -930,6 +939,10 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   // loop starts at the tile holding it), keys from lo_all on from none
   const int lo_key = WIN ? max(0, prefix + (DENSE ? row0 / G : 0) - a.window) : 0;
   const int lo_all = WIN && DENSE ? prefix + min(nq - 1, (row0 + C::ROWS - 1) / G) - a.window : lo_key;
+  // this workgroup's keys: split sp of the block's tile-aligned key range
+  int k_lo = lo_key & ~(kTile - 1), k_hi = kv_end;
+  split_range(a, sp, kv_end, k_lo, k_hi);
+  if (a.splits > 1 && k_lo >= k_hi) return;  // no partial (the combine counts the splits with keys)
 
   const int r = row0 + wave * 32 + j;
   const int pos = r / G;
@@ -1007,13 +1020,6 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   const uint32_t hkv = (uint32_t)a.num_kv_heads;
   const int32_t* bt_row = a.block_table + (int64_t)b * a.bt_stride;
 
-  // this workgroup's keys: split sp of the block's tile-aligned key range
-  int k_lo = lo_key & ~(kTile - 1), k_hi = kv_end;
-  if (a.splits > 1) {
-    const int chunk = ((max(0, kv_end - k_lo) + a.splits - 1) / a.splits + kTile - 1) & ~(kTile - 1);
-    k_lo += sp * chunk;
-    k_hi = min(kv_end, k_lo + chunk);
-  }
   // A wave whose 32 rows are all past the query count (a short draft tree,
   // the last block of a chunk) takes part in the tile loads, conversions and
   // barriers only; its rows are written as zeros.  The key loop is
@@ -1345,8 +1351,9 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   const float l_tot = sum_x32(l_run);
   // ---- split: this wave's unnormalized rows to the partials ----
   if (a.splits > 1) {
+    if (!wave_live) return;  // (no row of the wave is read back)
     const int rl = wave * 32 + j;
-    float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * C::ROWS + rl) * (D + 4);
+    float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * a.part_rows + rl) * (D + 4);
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
 #pragma unroll
@@ -1429,16 +1436,20 @@ __global__ __launch_bounds__(kCombineThreads) void verify_combine_kernel(VerifyA
     *op = half4_t{0, 0, 0, 0};
     return;
   }
-  const int S = a.splits;
-  const int64_t stride = (int64_t)ROWS * (D + 4);  // between splits of one row
-  const float* row = a.part + ((int64_t)pq * S * ROWS + rl) * (D + 4);
-  // one pass, 32 partials in flight: the running max rises batch by batch and
-  // rescales what is summed so far (a split count of 64 reads in 2 rounds)
-  constexpr int U = 32;
+  // the splits that hold keys of this block (the kernels' range)
+  const int prefix = max(0, a.prefix_lens[b]);
+  const int end = min(prefix + (a.tree_mask ? nq : min(nq, (qb * ROWS + ROWS + G - 1) / G)), a.max_context_len);
+  const int k_lo = a.window > 0 ? max(0, prefix - a.window) & ~(kTile - 1) : 0;
+  const int S = min(a.splits, (max(0, end - k_lo) + a.split_keys - 1) / a.split_keys);
+  const int64_t stride = (int64_t)a.part_rows * (D + 4);  // between splits of one row
+  const float* row = a.part + ((int64_t)pq * a.splits * a.part_rows + rl) * (D + 4);
+  // one pass: the running max rises batch by batch and rescales what is
+  // summed so far
   float M = -__builtin_inff();
   float4_t num = float4_t{0.f, 0.f, 0.f, 0.f};
   float den = 0.0f;
-  for (int s0 = 0; s0 < S; s0 += U) {
+  auto batch = [&](int s0, auto u_tag) {  // partials s0 .. s0 + U - 1, all in flight
+    constexpr int U = decltype(u_tag)::value;
     float m[U], l[U];
     float4_t x[U];
 #pragma unroll
@@ -1449,7 +1460,7 @@ __global__ __launch_bounds__(kCombineThreads) void verify_combine_kernel(VerifyA
       l[u] = pr[D + 1];
       x[u] = *reinterpret_cast<const float4_t*>(pr + 4 * c4);
     }
-    float mb = M;  // (partial maxima are finite: a split without keys keeps its initial max)
+    float mb = M;  // (partial maxima are finite: a split without visible keys keeps its initial max)
 #pragma unroll
     for (int u = 0; u < U; ++u) mb = s0 + u < S ? fmaxf(mb, m[u]) : mb;
     const float c = __builtin_amdgcn_exp2f(M - mb);  // 0 on the first batch
@@ -1462,6 +1473,13 @@ __global__ __launch_bounds__(kCombineThreads) void verify_combine_kernel(VerifyA
       den += f * l[u];
     }
     M = mb;
+  };
+  // 32 in flight for a long row cut for a batch of one (64 splits: 2 rounds),
+  // 8 for the few splits of a row in a full batch
+  if (S > 8) {
+    for (int s0 = 0; s0 < S; s0 += 32) batch(s0, std::integral_constant<int, 32>{});
+  } else if (S > 0) {
+    batch(0, std::integral_constant<int, 8>{});
   }
   const float inv = den > 0.0f ? 1.0f / den : 0.0f;
   half4_t o;
@@ -1573,34 +1591,51 @@ struct FreshDrafts {
   int64_t v_stride[3];
 };
 
-// Key-range split of the paged verify.  A launch with fewer workgroups than
-// the GPU keeps resident (two per CU) leaves CUs idle for the whole call --
-// batch-1 speculative decoding with a long context is the common case -- so
-// each (sequence, KV head, query block) is split until about that many
-// exist, down to kMinSplitKeys keys per split (512: a 32K-key batch-1 tree
-// verify at 8 KV heads fills all 512 slots, 4-5 % faster than 32 splits of
-// 1024 keys; a second round of splits is slower again); and one workgroup
-// never accumulates more than kMaxSplitKeys keys, which bounds the rounding
-// of its fp32 sums.  s8kv_verify_set_splits overrides the count (diagnostics).
+// Key-range split of the paged verify: the units of a (sequence, KV head,
+// query block) take an equal number of keys, so a short row has fewer of them
+// and the longest row's share bounds the launch.  Two reasons to split:
+//  * a launch with fewer workgroups than the GPU keeps resident leaves CUs
+//    idle for the whole call -- batch-1 speculative decoding with a long context
+//    is the common case -- so units are split until about that many exist,
+//    down to kMinSplitKeys keys per split (512: a 32K-key batch-1 tree verify
+//    at 8 KV heads fills all 512 slots, 4-5 % faster than 32 splits of 1024
+//    keys; a second round of splits is slower again);
+//  * rows of different lengths: with whole rows (or halves of each) the
+//    longest one runs alone at the end.  Splits of at least kMinSplitKeys keys,
+//    and 32 keys per query row (a split writes and the combine reads 1 KB a
+//    row, against the 270 bytes a key and head that it streams), up to
+//    kBalanceRounds units per resident workgroup, keep every CU busy.  Batch
+//    32, 5 queries, 8 KV heads, contexts of 256 .. 8,192 (mean 2,300): 2
+//    halves of each row 184.7 us a call, equal splits of 640 keys 132.9.
+// One workgroup never accumulates more than kMaxSplitKeys keys, which bounds
+// the rounding of its fp32 sums.  s8kv_verify_set_splits overrides the count
+// (diagnostics).
 constexpr int kMinSplitKeys = 512;
+constexpr int kBalanceRounds = 8;
 constexpr int kMaxSplitKeys = 1 << 20;
 constexpr int kMaxSplits = 1024;
 static std::atomic<int> g_verify_splits{0};  // 0: planned per call
-static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int keys, bool k8v3, bool wide, int rows) {
+static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int keys, bool k8v3, bool wide, int rows,
+                              int rows_wg) {
   const int64_t natural = (int64_t)batch * num_kv_heads * n_qblocks;
   const int64_t resident = (int64_t)verify::wg_per_cu(k8v3, wide, rows) * device_cus();
   int64_t s = natural < resident ? (resident + natural - 1) / natural : 1;
   s = std::min<int64_t>(s, std::max(1, keys / kMinSplitKeys));
+  if (batch > 1) {
+    const int64_t least = std::max(kMinSplitKeys, 32 * std::min(rows, rows_wg));
+    s = std::max(s, std::min(keys / least, (kBalanceRounds * resident + natural - 1) / natural));
+  }
   s = std::max<int64_t>(s, ((int64_t)keys + kMaxSplitKeys - 1) / kMaxSplitKeys);
   const int forced = g_verify_splits.load();
   if (forced > 0) s = forced;
   return (int)std::max<int64_t>(1, std::min<int64_t>(s, kMaxSplits));
 }
-static int64_t verify_part_bytes(int batch, int num_kv_heads, int n_qblocks, int head_dim, int splits, bool k8v3,
-                                 bool wide, int rows) {
+// Rows of a unit's partials: whole 32-row groups of the rows a block can have.
+static int verify_part_rows(int rows, int rows_wg) { return std::min(rows_wg, (rows + 31) / 32 * 32); }
+static int64_t verify_part_bytes(int batch, int num_kv_heads, int n_qblocks, int head_dim, int splits, int rows,
+                                 int rows_wg) {
   if (splits <= 1) return 0;
-  return (int64_t)batch * num_kv_heads * n_qblocks * splits * verify::rows_per_wg(head_dim, k8v3, wide, rows) *
-         (head_dim + 4) * 4;
+  return (int64_t)batch * num_kv_heads * n_qblocks * splits * verify_part_rows(rows, rows_wg) * (head_dim + 4) * 4;
 }
 
 extern "C" int64_t s8kv_verify_workspace_size(int batch, int num_q_heads, int num_kv_heads, int head_dim,
@@ -1618,8 +1653,8 @@ extern "C" int64_t s8kv_verify_workspace_size(int batch, int num_q_heads, int nu
       const int n_qblocks = (rows + rows_wg - 1) / rows_wg;
       need = std::max(need, verify_part_bytes(batch, num_kv_heads, n_qblocks, head_dim,
                                               verify_plan_splits(batch, num_kv_heads, n_qblocks, max_context_len,
-                                                                 k8v3, wide, rows),
-                                              k8v3, wide, rows));
+                                                                 k8v3, wide, rows, rows_wg),
+                                              rows, rows_wg));
     }
   }
   return need;
@@ -1637,11 +1672,16 @@ static int verify_use_workspace(verify::VerifyArgs& a, int head_dim, bool k8v3, 
   const int keys = a.window > 0 ? (int)std::min<int64_t>(a.max_context_len, (int64_t)a.window + a.max_queries)
                                 : a.max_context_len;
   const int rows = a.group * a.max_queries;
-  const int s = verify_plan_splits(a.batch, a.num_kv_heads, a.n_qblocks, keys, k8v3, wide, rows);
-  const int64_t need = verify_part_bytes(a.batch, a.num_kv_heads, a.n_qblocks, head_dim, s, k8v3, wide, rows);
+  const int rows_wg = verify::rows_per_wg(head_dim, k8v3, wide, rows);
+  const int s = verify_plan_splits(a.batch, a.num_kv_heads, a.n_qblocks, keys, k8v3, wide, rows, rows_wg);
+  const int64_t need = verify_part_bytes(a.batch, a.num_kv_heads, a.n_qblocks, head_dim, s, rows, rows_wg);
   const bool fits = workspace != nullptr && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
   if (s > 1 && fits) {
     a.splits = s;
+    // (a window's range starts at the tile of its first key: up to kTile - 1 keys more)
+    const int64_t range = (int64_t)keys + verify::kTile - 1;
+    a.split_keys = (int)(((range + s - 1) / s + verify::kTile - 1) / verify::kTile * verify::kTile);
+    a.part_rows = verify_part_rows(rows, rows_wg);
     a.part = (float*)workspace;
   }
   S8KV_REQUIRE(fits || keys <= kMaxSplitKeys, S8KV_ERR_WORKSPACE,
