@@ -1020,333 +1020,533 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   const uint32_t hkv = (uint32_t)a.num_kv_heads;
   const int32_t* bt_row = a.block_table + (int64_t)b * a.bt_stride;
 
+  // window verify with fresh drafts: whether the tile at `base` holds draft
+  // keys (wave-uniform), whose K then has a low fp16 part, and the draft
+  // index of its key tt (-1: a prefix key, or no fresh drafts)
+  auto fresh_tile = [&](int base) -> bool {
+    if constexpr (FRESH) return base + kTile > prefix && base < prefix + nq;
+    return false;
+  };
+  auto fresh_draft = [&](int base, int tt) -> int {
+    if constexpr (FRESH) {
+      const int di = base + tt - prefix;
+      return (di >= 0 && di < nq) ? di : -1;
+    }
+    return -1;
+  };
+
+  // ---- registers -> LDS: 16 dims of one key (K or V), fp16 ----
+  auto store16 = [&](char* dst, u32x4_t d) {  // 16 int8
+    *reinterpret_cast<half8_t*>(dst) = i8x8_to_f16(u32x2_t{d.x, d.y});
+    *reinterpret_cast<half8_t*>(dst + 16) = i8x8_to_f16(u32x2_t{d.z, d.w});
+  };
+  auto store_k = [&](int buf, int base, int tt, int part, u32x4_t d) {
+    char* kb = smem + buf * C::BUF + tt * C::KROW + part * 32;
+    [[maybe_unused]] char* klo = smem + C::KLO_OFF + buf * C::KBYTES + tt * C::KROW + part * 32;
+    const int di = fresh_draft(base, tt);
+    if (di >= 0) {  // the draft's fresh values as fp16 hi + lo
+      const float4_t* kp = reinterpret_cast<const float4_t*>(
+          a.kd + (int64_t)b * a.kd_stride_b + (int64_t)di * a.kd_stride_s + (int64_t)h * a.kd_stride_h + part * 16);
+      const float4_t kx[4] = {kp[0], kp[1], kp[2], kp[3]};  // (rows 16-byte aligned: checked on the host)
+      half8_t k0, k1, l0, l1;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x0 = kx[e >> 2][e & 3], x1 = kx[2 + (e >> 2)][e & 3];
+        k0[e] = (_Float16)x0;
+        k1[e] = (_Float16)x1;
+        l0[e] = (_Float16)(x0 - (float)k0[e]);
+        l1[e] = (_Float16)(x1 - (float)k1[e]);
+      }
+      *reinterpret_cast<half8_t*>(klo) = l0;
+      *reinterpret_cast<half8_t*>(klo + 16) = l1;
+      *reinterpret_cast<half8_t*>(kb) = k0;
+      *reinterpret_cast<half8_t*>(kb + 16) = k1;
+      return;
+    }
+    if (fresh_tile(base)) {  // a prefix key in a tile holding drafts: no low part
+      *reinterpret_cast<half8_t*>(klo) = half8_t{};
+      *reinterpret_cast<half8_t*>(klo + 16) = half8_t{};
+    }
+    store16(kb, d);
+  };
+  // (K8V3: d holds a code group's three words; vt's half of its 32 values)
+  auto store_v = [&](int buf, int base, int tt, int vt, u32x4_t d) {
+    char* vb = smem + buf * C::BUF + C::KBYTES + tt * C::VROW;
+    const int di = fresh_draft(base, tt);
+    if (di >= 0) {
+      const int part = vt & 7;
+      const half8_t* vp = reinterpret_cast<const half8_t*>(
+          a.vd + (int64_t)b * a.vd_stride_b + (int64_t)di * a.vd_stride_s + (int64_t)h * a.vd_stride_h + part * 16);
+      *reinterpret_cast<half8_t*>(vb + part * 32) = vp[0];
+      *reinterpret_cast<half8_t*>(vb + part * 32 + 16) = vp[1];
+      return;
+    }
+    if constexpr (!K8V3) {
+      store16(vb + (vt & 7) * 32, d);
+    } else {  // 16 codes of one group -> fp16 codebook entries
+      const int gi = (vt >> 1) & 3, sh = (vt & 1) * 16;
+      const uint32_t w0 = d.x >> sh, w1 = d.y >> sh, w2 = d.z >> sh;
+      char* dst = vb + gi * 64 + sh * 2;
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4 += 2) {
+        u32x4_t o;
+        const uint32_t sel0 = spread4(w0 >> (4 * q4)) | (spread4(w1 >> (4 * q4)) << 1) | (spread4(w2 >> (4 * q4)) << 2);
+        const uint32_t sel1 =
+            spread4(w0 >> (4 * q4 + 4)) | (spread4(w1 >> (4 * q4 + 4)) << 1) | (spread4(w2 >> (4 * q4 + 4)) << 2);
+        const u32x2_t r0 = codebook_lookup4(sel0, tlo03, tlo47, thi03, thi47);
+        const u32x2_t r1 = codebook_lookup4(sel1, tlo03, tlo47, thi03, thi47);
+        o.x = r0.x; o.y = r0.y; o.z = r1.x; o.w = r1.y;
+        *reinterpret_cast<u32x4_t*>(dst + q4 * 8) = o;
+      }
+    }
+  };
+  // a V scale is staged finite (NaN and inf -> 2^100): the weight of a hidden
+  // key, exp2(-inf) * scale, is then 0 whatever was stored there (clamped
+  // here, where the load is consumed, not where it is issued); a fresh
+  // draft's K and V scales are 1
+  auto store_scale = [&](int buf, int base, int tt, bool k_side, float v) {
+    float* sb = reinterpret_cast<float*>(smem + buf * C::BUF + C::KBYTES + C::VBYTES);
+    sb[k_side ? tt : kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : k_side ? v : fminf(v, 0x1p100f);
+  };
+
+  // ---- one 32-key tile from LDS buffer `buf`: scores, weights, PV ----
+  float16_t sc;
+  u32x4_t wh[2], wl[2];  // weights of keys 16t .. 16t + 15 as fp16 hi + lo
+  auto read_ka = [&](int buf, int m) -> half8_t {
+    return *reinterpret_cast<const half8_t*>(smem + buf * C::BUF + j * C::KROW + hf * 128 + 16 * m);
+  };
+  auto qk = [&](int buf) {
+    half8_t ka[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) ka[m] = read_ka(buf, m);
+    sc = float16_t{};
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      sc = mfma32x32x16(ka[m], qhi[m], sc);
+      if constexpr (!DENSE) sc = mfma32x32x16(ka[m], qlo[m], sc);
+    }
+  };
+  auto qk_fresh = [&](int buf, int base) {
+    if constexpr (FRESH) {  // fresh draft keys: K = hi + lo
+      if (fresh_tile(base)) {
+        const char* lrow = smem + C::KLO_OFF + buf * C::KBYTES + j * C::KROW + hf * 128;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) sc = mfma32x32x16(*reinterpret_cast<const half8_t*>(lrow + 16 * m), qhi[m], sc);
+      }
+    }
+  };
+  // Only the scores depend on the tile's kind (keys hidden from some row:
+  // masked, as -inf); the rescale, the weights and the PV are one code path
+  // for every tile, so the accumulators keep their registers throughout.
+  // (dense: the K "scales" are the softmax scale, the V scales 1)
+  auto weights = [&](int buf, int base, bool masked) {
+    const float* sb = reinterpret_cast<const float*>(smem + buf * C::BUF + C::KBYTES + C::VBYTES);
+    // this lane's keys: register r is key 8 (r / 4) + 4 hf + r % 4
+    float4_t ks4[DENSE ? 1 : 4];
+    if constexpr (!DENSE) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ks4[q] = *reinterpret_cast<const float4_t*>(sb + 8 * q + 4 * hf);
+    }
+    auto kscale = [&](int rr) -> float {
+      if constexpr (DENSE) return a.qscale;
+      else return ks4[rr >> 2][rr & 3];
+    };
+    float y[16];  // score relative to the running max, log2 domain; -inf: hidden from this row
+#pragma unroll
+    for (int rr = 0; rr < 16; ++rr) y[rr] = __builtin_fmaf(sc[rr], kscale(rr), -m_ref);
+    if (masked) {
+      // bit i: tile key i is visible to this row
+      auto below = [](int n) -> uint32_t { return n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u; };
+      uint32_t vis;
+      if (tree) {  // the prefix keys, and the drafts whose bits are set (none past the 64th)
+        const int d0 = base - prefix;  // draft index of tile key 0
+        vis = d0 >= 64 ? 0u : d0 >= 0 ? (uint32_t)(tmask >> d0) : below(-d0) | (d0 > -32 ? (uint32_t)tmask << -d0 : 0u);
+      } else {
+        vis = below(prefix + pos + 1 - base);
+      }
+      vis &= below(row_live ? kv_end - base : 0);
+      if constexpr (WIN) vis &= ~below((DENSE ? prefix + pos - a.window : lo_key) - base);
+      vis >>= 4 * hf;
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) y[rr] = (vis >> (8 * (rr >> 2) + (rr & 3))) & 1u ? y[rr] : kNegInf;
+    }
+    float my = y[0];
+#pragma unroll
+    for (int rr = 1; rr < 16; ++rr) my = fmaxf(my, y[rr]);
+    my = max_x32(my);
+    // V-scale bound test: lane l checks the V scale of key l % 32 (paged
+    // window: not of the keys below it, which may hold anything)
+    float vp = 0.0f;
+    if constexpr (!DENSE) vp = sb[kTile + j];
+    if constexpr (WIN && !DENSE) vp = base + j >= lo_key ? vp : 0.0f;
+    if (__builtin_amdgcn_ballot_w64(my > ws.thr() || vp > ws.vbound()) != 0) {
+      // rare: a V scale above the bound lowers the weight shift (by d, a
+      // power of two folded into alpha), or a score passes the lazy slack:
+      // the running max rises to the tile's (from the products, exactly),
+      // l and the accumulators are rescaled, the scores re-referenced
+      int d = 0;
+      if (__builtin_amdgcn_ballot_w64(vp > ws.vbound()) != 0) {
+        float vmx = fmaxf(vp, shfl_xor_f(vp, 1));
+        vmx = fmaxf(vmx, shfl_xor_f(vmx, 2));
+        vmx = fmaxf(vmx, shfl_xor_f(vmx, 4));
+        vmx = fmaxf(vmx, shfl_xor_f(vmx, 8));
+        d = ws.raise(max_x16(vmx), kMaxSlack);
+      }
+      m_ref -= (float)d;
+      float mt = kNegInf;
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) mt = fmaxf(mt, y[rr] != kNegInf ? sc[rr] * kscale(rr) : kNegInf);
+      mt = max_x32(mt);
+      const float m_new = fmaxf(m_ref, mt - (float)ws.esh);
+      const float alpha = __builtin_amdgcn_exp2f(m_ref - m_new) * __builtin_ldexpf(1.0f, d);
+      l_run *= alpha;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[n] *= alpha;  // (plain VALU: its MFMA hazards are the compiler's)
+      m_ref = m_new;
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) y[rr] = y[rr] != kNegInf ? __builtin_fmaf(sc[rr], kscale(rr), -m_new) : kNegInf;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      // weights p * (V scale | block norm) of keys 16t .. 16t + 15 as fp16
+      // hi + lo (hi: the top 11 significant bits, exact in fp16 over its
+      // normal range; lo: the rest); hidden keys weigh 0 whatever their
+      // scale (inf and NaN included)
+      float4_t vs0{}, vs1{};
+      if constexpr (!DENSE) {
+        vs0 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 4 * hf);
+        vs1 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 8 + 4 * hf);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        float w[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int rr = 8 * t + e + u;
+          const float ev = __builtin_amdgcn_exp2f(y[rr]);  // 0 for hidden keys
+          l_run += ev;
+          // (finite scales: 0 for hidden keys; dense: ev itself, which
+          // split_pair's rounding reads before its asm does)
+          if constexpr (DENSE) w[u] = ev;
+          else w[u] = ev * (e + u < 4 ? vs0[e + u] : vs1[e + u - 4]);
+        }
+        uint32_t hw, lw;
+        split_pair(w[0], w[1], hw, lw);
+        wh[t][e / 2] = hw;
+        wl[t][e / 2] = lw;
+      }
+    }
+  };
+  // V^T operands of keys 16t .. 16t + 15 by transpose reads; lane (li, group
+  // G) reads row 16t + 4 hf + li / 4 (+ 8), dims 32 n + 16 (G & 1) + 4 (li % 4)
+  // .. + 3
+  auto read_va = [&](int buf, int t, int n) -> half8_t {
+    const int li = lane & 15;
+    const char* src = smem + buf * C::BUF + C::KBYTES + (16 * t + 4 * hf + (li >> 2)) * C::VROW +
+                      (16 * ((lane >> 4) & 1) + 4 * (li & 3)) * 2 + 64 * n;
+    const i16x4_t lw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((S8KV_LDS i16x4_t*)(src));
+    const i16x4_t hw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((S8KV_LDS i16x4_t*)(src + 8 * C::VROW));
+    const half4_t l4 = __builtin_bit_cast(half4_t, lw), h4 = __builtin_bit_cast(half4_t, hw);
+    return half8_t{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
+  };
+  auto pv = [&](int buf) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const half8_t pbh = __builtin_bit_cast(half8_t, wh[t]), pbl = __builtin_bit_cast(half8_t, wl[t]);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const half8_t va = read_va(buf, t, n);
+        acc[n] = mfma32x32x16(va, pbh, acc[n]);
+        acc[n] = mfma32x32x16(va, pbl, acc[n]);
+      }
+    }
+  };
+  // a tile is masked when it reaches keys that some row of the block does
+  // not see, or the end of the visible keys (wave-uniform)
+  auto hides = [&](int base) -> bool {
+    return !(base + kTile <= vis_all && base + kTile <= kv_end && (!WIN || base >= lo_all));
+  };
+
   // A wave whose 32 rows are all past the query count (a short draft tree,
   // the last block of a chunk) takes part in the tile loads, conversions and
   // barriers only; its rows are written as zeros.  The key loop is
   // instantiated for both kinds of wave, so neither carries the other's branch.
   const bool wave_live = (row0 + wave * 32) / G < nq;
   auto key_loop = [&](auto live_tag) {
-  constexpr bool LIVE = decltype(live_tag)::value;
-  for (int u0 = k_lo; u0 < k_hi; u0 += kSubKeys) {
-    const int u1 = min(k_hi, u0 + kSubKeys);
-    const int fb = u0 >> bs_log2;
-    const int nblk = ((u1 - 1) >> bs_log2) - fb + 1;
-    __syncthreads();  // previous users of bt_lds and the tile buffers are done
-    if constexpr (!DENSE)
-      for (int i = tid; i < nblk; i += C::THREADS) bt_lds[i] = bt_row[fb + i];
-    __syncthreads();
-
-    auto row_of = [&](int kk) -> uint32_t {
-      kk = min(kk, u1 - 1);
-      const uint32_t blk = (uint32_t)bt_lds[(kk >> bs_log2) - fb];
-      return ((blk * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)kk & bsm);
-    };
-
-    // window verify with fresh drafts: whether the tile at `base` holds draft
-    // keys (wave-uniform), whose K then has a low fp16 part, and the draft
-    // index of its key tt (-1: a prefix key, or no fresh drafts)
-    auto fresh_tile = [&](int base) -> bool {
-      if constexpr (FRESH) return base + kTile > prefix && base < prefix + nq;
-      return false;
-    };
-    auto fresh_draft = [&](int base, int tt) -> int {
-      if constexpr (FRESH) {
-        const int di = base + tt - prefix;
-        return (di >= 0 && di < nq) ? di : -1;
-      }
-      return -1;
-    };
-    // dense: 512 16-byte fp16 K chunks and as many V chunks per tile, two
-    // each per thread of a 4-wave workgroup, one of an 8-wave one
-    constexpr int NCH = DENSE ? 512 / C::THREADS : 1;
-    struct TileRegs {
-      u32x4_t k[NCH], v[NCH];
-      float s;
-    };
-    // one 16-byte K chunk and one V chunk (K8V3: a half code group's three
-    // words) per thread, and the tile's 2 x 32 scales in threads 0..63
-    // (the cache rows of fresh drafts are loaded too, and not used)
-    auto load_tile = [&](TileRegs& R, int base) {
-      if constexpr (DENSE) {  // fp16 rows of keys base .. base + 31 (clamped to the last key)
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-          const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
-          const int64_t tok = k0 + min(base + tt, nk - 1);
-          R.k[i] = *reinterpret_cast<const u32x4_t*>(a.k_f16 + tok * a.k_stride_t + h * a.k_stride_h + part * 8);
-          R.v[i] = *reinterpret_cast<const u32x4_t*>(a.v_f16 + tok * a.v_stride_t + h * a.v_stride_h + part * 8);
-        }
-        R.s = 1.0f;
-        return;
-      }
-      // 4 waves: every thread one K and one V chunk; 8 waves: threads 0..255
-      // the K chunks, 256..511 the V chunks (vt: the V job index)
-      constexpr bool SPLITKV = C::WAVES == 8;
-      const bool kthr = !SPLITKV || tid < 256, vthr = !SPLITKV || tid >= 256;
-      const int vt = tid & 255;
-      const int tt = tid >> 3 & 31, part = tid & 7;
-      const uint32_t row = row_of(base + tt);
-      if (kthr) R.k[0] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
-      if (!vthr) {
-      } else if constexpr (K8V3) {
-        const int grp = vt >> 1;
-        const int gt = grp / C::NG, gi = grp % C::NG;
-        const uint32_t off = row_of(base + gt) * (uint32_t)(C::WORDS * 4) + (uint32_t)gi * 12u;
-        const u32x3_t w = bload96(vc, off);
-        R.v[0].x = w.x;
-        R.v[0].y = w.y;
-        R.v[0].z = w.z;
-      } else {
-        R.v[0] = bload128(vc, row * (uint32_t)D + (uint32_t)part * 16u);
-      }
-      // (two loads, each with one descriptor: a descriptor chosen per lane
-      // would be issued lane by lane)
-      if (tid < kTile) R.s = __builtin_bit_cast(float, bload32(ks, row_of(base + tid) * 4u));
-      else if (tid < 2 * kTile) R.s = __builtin_bit_cast(float, bload32(vs, row_of(base + tid - kTile) * 4u));
-    };
-    auto store_tile = [&](const TileRegs& R, int buf, int base) {
-      char* kb = smem + buf * C::BUF;
-      char* vb = kb + C::KBYTES;
-      float* sb = reinterpret_cast<float*>(vb + C::VBYTES);
-      if constexpr (DENSE) {  // fp16 rows as they are; K "scales" carry the softmax scale, V scales are 1
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-          const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
-          *reinterpret_cast<u32x4_t*>(kb + tt * C::KROW + part * 16) = R.k[i];
-          *reinterpret_cast<u32x4_t*>(vb + tt * C::VROW + part * 16) = R.v[i];
-        }
-        if (tid < 2 * kTile) sb[tid] = tid < kTile ? a.qscale : 1.0f;
-        return;
-      }
-      constexpr bool SPLITKV = C::WAVES == 8;
-      const bool kthr = !SPLITKV || tid < 256, vthr = !SPLITKV || tid >= 256;
-      const int vt = tid & 255;
-      const int tt = tid >> 3 & 31, part = tid & 7;
-      const int di = kthr ? fresh_draft(base, tt) : -1;
-      if (!kthr) {
-      } else if (di >= 0) {  // the draft's fresh values, dims part*16 .. +16: K as fp16 hi + lo, V as it is
-        const float4_t* kp = reinterpret_cast<const float4_t*>(
-            a.kd + (int64_t)b * a.kd_stride_b + (int64_t)di * a.kd_stride_s + (int64_t)h * a.kd_stride_h + part * 16);
-        const _Float16* vp = a.vd + (int64_t)b * a.vd_stride_b + (int64_t)di * a.vd_stride_s +
-                             (int64_t)h * a.vd_stride_h + part * 16;
-        const float4_t kx[4] = {kp[0], kp[1], kp[2], kp[3]};  // (rows 16-byte aligned: checked on the host)
-        half8_t k0, k1, l0, l1;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x0 = kx[e >> 2][e & 3], x1 = kx[2 + (e >> 2)][e & 3];
-          k0[e] = (_Float16)x0;
-          k1[e] = (_Float16)x1;
-          l0[e] = (_Float16)(x0 - (float)k0[e]);
-          l1[e] = (_Float16)(x1 - (float)k1[e]);
-        }
-        char* klo = smem + C::KLO_OFF + buf * C::KBYTES + tt * C::KROW + part * 32;
-        *reinterpret_cast<half8_t*>(klo) = l0;
-        *reinterpret_cast<half8_t*>(klo + 16) = l1;
-        *reinterpret_cast<half8_t*>(kb + tt * C::KROW + part * 32) = k0;
-        *reinterpret_cast<half8_t*>(kb + tt * C::KROW + part * 32 + 16) = k1;
-        *reinterpret_cast<half8_t*>(vb + tt * C::VROW + part * 32) = *reinterpret_cast<const half8_t*>(vp);
-        *reinterpret_cast<half8_t*>(vb + tt * C::VROW + part * 32 + 16) = *reinterpret_cast<const half8_t*>(vp + 8);
-      } else {
-        if (fresh_tile(base)) {  // a prefix key in a tile holding drafts: no low part
-          char* klo = smem + C::KLO_OFF + buf * C::KBYTES + tt * C::KROW + part * 32;
-          *reinterpret_cast<half8_t*>(klo) = half8_t{};
-          *reinterpret_cast<half8_t*>(klo + 16) = half8_t{};
-        }
-        *reinterpret_cast<half8_t*>(kb + tt * C::KROW + part * 32) = i8x8_to_f16(u32x2_t{R.k[0].x, R.k[0].y});
-        *reinterpret_cast<half8_t*>(kb + tt * C::KROW + part * 32 + 16) = i8x8_to_f16(u32x2_t{R.k[0].z, R.k[0].w});
-      }
-      // int8 V rows: by the V threads (the same key and part as a K thread's
-      // tt, part; a fresh draft's V is written above with its K)
-      if constexpr (!K8V3) {
-        if (vthr && fresh_draft(base, tt) < 0) {
-          *reinterpret_cast<half8_t*>(vb + tt * C::VROW + part * 32) = i8x8_to_f16(u32x2_t{R.v[0].x, R.v[0].y});
-          *reinterpret_cast<half8_t*>(vb + tt * C::VROW + part * 32 + 16) = i8x8_to_f16(u32x2_t{R.v[0].z, R.v[0].w});
-        }
-      }
-      if constexpr (K8V3) {  // 16 codes of one group -> fp16 codebook entries (prefix keys)
-        const int grp = vt >> 1, half = vt & 1;
-        const int gt = grp / C::NG, gi = grp % C::NG;
-        if (vthr && fresh_draft(base, gt) < 0) {
-          const int sh = half * 16;
-          const uint32_t w0 = R.v[0].x >> sh, w1 = R.v[0].y >> sh, w2 = R.v[0].z >> sh;
-          char* dst = vb + gt * C::VROW + gi * 64 + sh * 2;
-#pragma unroll
-          for (int q4 = 0; q4 < 4; q4 += 2) {
-            u32x4_t o;
-            const uint32_t sel0 =
-                spread4(w0 >> (4 * q4)) | (spread4(w1 >> (4 * q4)) << 1) | (spread4(w2 >> (4 * q4)) << 2);
-            const uint32_t sel1 = spread4(w0 >> (4 * q4 + 4)) | (spread4(w1 >> (4 * q4 + 4)) << 1) |
-                                  (spread4(w2 >> (4 * q4 + 4)) << 2);
-            const u32x2_t r0 = codebook_lookup4(sel0, tlo03, tlo47, thi03, thi47);
-            const u32x2_t r1 = codebook_lookup4(sel1, tlo03, tlo47, thi03, thi47);
-            o.x = r0.x; o.y = r0.y; o.z = r1.x; o.w = r1.y;
-            *reinterpret_cast<u32x4_t*>(dst + q4 * 8) = o;
-          }
-        }
-      }
-      // a V scale is staged finite (NaN and inf -> 2^100): the weight of a
-      // hidden key, exp2(-inf) * scale, is then 0 whatever was stored there
-      // (clamped here, where the load is consumed, not where it is issued);
-      // a fresh draft's K and V scales are 1
-      if (tid < 2 * kTile)
-        sb[tid] = fresh_draft(base, tid & (kTile - 1)) >= 0 ? 1.0f : tid < kTile ? R.s : fminf(R.s, 0x1p100f);
-    };
-
-    // ---- one 32-key tile from LDS buffer `buf` ----
-    // Only the scores depend on the tile's kind (keys hidden from some row:
-    // masked, as -inf); the rescale, the weights and the PV are one code path
-    // for every tile, so the accumulators keep their registers throughout.
-    auto process = [&](int buf, int base, bool masked) {
-      const char* kb = smem + buf * C::BUF;
-      const char* vb = kb + C::KBYTES;
-      const float* sb = reinterpret_cast<const float*>(vb + C::VBYTES);
-      float16_t sc = float16_t{};
-      {
-        const char* krow = kb + j * C::KROW + hf * 128;
-        half8_t ka[8];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) ka[m] = *reinterpret_cast<const half8_t*>(krow + 16 * m);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          sc = mfma32x32x16(ka[m], qhi[m], sc);
-          if constexpr (!DENSE) sc = mfma32x32x16(ka[m], qlo[m], sc);
-        }
-      }
-      if constexpr (FRESH) {  // fresh draft keys: K = hi + lo
-        if (fresh_tile(base)) {
-          const char* lrow = smem + C::KLO_OFF + buf * C::KBYTES + j * C::KROW + hf * 128;
-#pragma unroll
-          for (int m = 0; m < 8; ++m) sc = mfma32x32x16(*reinterpret_cast<const half8_t*>(lrow + 16 * m), qhi[m], sc);
-        }
-      }
-      // this lane's keys: register r is key 8 (r / 4) + 4 hf + r % 4
-      float4_t ks4[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) ks4[q] = *reinterpret_cast<const float4_t*>(sb + 8 * q + 4 * hf);
-      auto kscale = [&](int rr) -> float { return ks4[rr >> 2][rr & 3]; };
-      float y[16];  // score relative to the running max, log2 domain; -inf: hidden from this row
-      if (masked) {
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-          const int kk = base + 8 * (rr >> 2) + 4 * hf + (rr & 3);
-          const int di = kk - prefix;
-          const bool dvis = tree ? ((uint32_t)di < 64u && ((tmask >> (di & 63)) & 1ull)) : di <= pos;
-          const bool vis = kk < kv_end && row_live && (di < 0 || dvis) &&
-                           (!WIN || kk >= (DENSE ? prefix + pos - a.window : lo_key));
-          const float v = __builtin_fmaf(sc[rr], kscale(rr), -m_ref);
-          y[rr] = vis ? v : kNegInf;
-        }
-      } else {
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) y[rr] = __builtin_fmaf(sc[rr], kscale(rr), -m_ref);
-      }
-      float my = y[0];
-#pragma unroll
-      for (int rr = 1; rr < 16; ++rr) my = fmaxf(my, y[rr]);
-      my = max_x32(my);
-      // V-scale bound test: lane l checks the V scale of key l % 32 (paged
-      // window: not of the keys below it, which may hold anything)
-      float vp = sb[kTile + j];
-      if constexpr (WIN && !DENSE) vp = base + j >= lo_key ? vp : 0.0f;
-      if (__builtin_amdgcn_ballot_w64(my > ws.thr() || vp > ws.vbound()) != 0) {
-        // rare: a V scale above the bound lowers the weight shift (by d, a
-        // power of two folded into alpha), or a score passes the lazy slack:
-        // the running max rises to the tile's (from the products, exactly),
-        // l and the accumulators are rescaled, the scores re-referenced
-        int d = 0;
-        if (__builtin_amdgcn_ballot_w64(vp > ws.vbound()) != 0) {
-          float vmx = fmaxf(vp, shfl_xor_f(vp, 1));
-          vmx = fmaxf(vmx, shfl_xor_f(vmx, 2));
-          vmx = fmaxf(vmx, shfl_xor_f(vmx, 4));
-          vmx = fmaxf(vmx, shfl_xor_f(vmx, 8));
-          d = ws.raise(max_x16(vmx), kMaxSlack);
-        }
-        m_ref -= (float)d;
-        float mt = kNegInf;
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) mt = fmaxf(mt, y[rr] != kNegInf ? sc[rr] * kscale(rr) : kNegInf);
-        mt = max_x32(mt);
-        const float m_new = fmaxf(m_ref, mt - (float)ws.esh);
-        const float alpha = __builtin_amdgcn_exp2f(m_ref - m_new) * __builtin_ldexpf(1.0f, d);
-        l_run *= alpha;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) acc[n] *= alpha;  // (plain VALU: its MFMA hazards are the compiler's)
-        m_ref = m_new;
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) y[rr] = y[rr] != kNegInf ? __builtin_fmaf(sc[rr], kscale(rr), -m_new) : kNegInf;
-      }
-      const int li = lane & 15;
-      const char* vrow = vb + (4 * hf + (li >> 2)) * C::VROW + (16 * ((lane >> 4) & 1) + 4 * (li & 3)) * 2;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        // weights p * (V scale | block norm) of keys 16t .. 16t + 15 as fp16
-        // hi + lo (hi: the top 11 significant bits, exact in fp16 over its
-        // normal range; lo: the rest); hidden keys weigh 0 whatever their
-        // scale (inf and NaN included)
-        const float4_t vs0 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 4 * hf);
-        const float4_t vs1 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 8 + 4 * hf);
-        u32x4_t hi4, lo4;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          float w[2];
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int rr = 8 * t + e + u;
-            const float ev = __builtin_amdgcn_exp2f(y[rr]);  // 0 for hidden keys
-            l_run += ev;
-            w[u] = ev * (e + u < 4 ? vs0[e + u] : vs1[e + u - 4]);  // (finite scales: 0 for hidden keys)
-          }
-          uint32_t hw, lw;
-          split_pair(w[0], w[1], hw, lw);
-          hi4[e / 2] = hw;
-          lo4[e / 2] = lw;
-        }
-        const half8_t pbh = __builtin_bit_cast(half8_t, hi4), pbl = __builtin_bit_cast(half8_t, lo4);
-        // PV: V^T operands by transpose reads; lane (li, group G) reads row
-        // 16t + 4 hf + li / 4 (+ 8), dims 32 n + 16 (G & 1) + 4 (li % 4) .. + 3
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-          const char* src = vrow + 16 * t * C::VROW + 64 * n;
-          const i16x4_t lw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((S8KV_LDS i16x4_t*)(src));
-          const i16x4_t hw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((S8KV_LDS i16x4_t*)(src + 8 * C::VROW));
-          const half4_t l4 = __builtin_bit_cast(half4_t, lw), h4 = __builtin_bit_cast(half4_t, hw);
-          const half8_t va = half8_t{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
-          acc[n] = mfma32x32x16(va, pbh, acc[n]);
-          acc[n] = mfma32x32x16(va, pbl, acc[n]);
-        }
-      }
-    };
-
-    // a tile is masked when it reaches keys that some row of the block does
-    // not see, or the end of the visible keys (wave-uniform)
-    auto compute = [&](int buf, int base) {
-      if constexpr (LIVE)
-        process(buf, base, !(base + kTile <= vis_all && base + kTile <= kv_end && (!WIN || base >= lo_all)));
-    };
-    const int ntiles = (u1 - u0 + kTile - 1) / kTile;
-    TileRegs ra, rb;
-    load_tile(ra, u0);
-    if (ntiles > 1) load_tile(rb, u0 + kTile);
-    store_tile(ra, 0, u0);
-    __syncthreads();
-    for (int t = 0; t < ntiles; t += 2) {  // (one exit: the accumulators keep their registers)
-      const int base = u0 + t * kTile;
-      if (t + 2 < ntiles) load_tile(ra, base + 2 * kTile);
-      compute(0, base);
-      if (t + 1 < ntiles) store_tile(rb, 1, base + kTile);
-      __syncthreads();
-      if (t + 1 < ntiles) {
-        if (t + 3 < ntiles) load_tile(rb, base + 3 * kTile);
-        compute(1, base + kTile);
-        if (t + 2 < ntiles) store_tile(ra, 0, base + 2 * kTile);
+    constexpr bool LIVE = decltype(live_tag)::value;
+    if constexpr (EIGHT) {
+      // The waves of a SIMD (wave w and w + 4) run half a tile apart: while
+      // waves 0..3 issue a tile's MFMAs (PV of tile t - 1, QK of tile t), waves
+      // 4..7 do the softmax of tile t - 1 and stage, then the other way
+      // round, a barrier between the halves.  In step, as one barrier a tile
+      // leaves them, both used the matrix cores and then the VALU at the same
+      // time.  With the scalar addresses below, us a call, before -> now:
+      // 16 x 512-query chunk over 4,096 keys 1,077 -> 1,024 (8 % fewer cycles, but the
+      // matrix cores then run the clock down: 2.13 -> 2.0 GHz; without any
+      // softmax or staging it would be 790, at 1.73 GHz); 32 trees of 16 to
+      // 64 nodes over 8,192 keys 448 -> 413; 12 ragged dense prompts 854 -> 751.
+      //   half 2t    : waves 0-3  PV(t-1), QK(t)          waves 4-7  softmax(t-1), V(t) -> LDS
+      //   half 2t + 1: waves 0-3  softmax(t), K(t+1) -> LDS   waves 4-7  PV(t-1), QK(t)
+      // K(t+1) replaces K(t-1), last read in half 2t - 1, and V(t) replaces
+      // V(t-2), last read (as PV of waves 4..7) in half 2t - 1; the scales of
+      // a tile, staged with it, are read up to half 2t + 2 and replaced in
+      // 2t + 3 (K) and 2t + 4 (V).
+      // Global loads run two tiles ahead into two register sets.
+      const bool kw = wave < 4;  // waves 0..3 stage K, waves 4..7 V
+      const int st = tid & 255;
+      const int tt = st >> 3, part = st & 7;
+      constexpr int NCH = DENSE ? 2 : 1;
+      struct HalfTile {
+        u32x4_t d[NCH];
+        float s;
+        int bid;  // block id of the tile loaded next into this set
+      };
+      // (Addresses are scalar but for constant lane offsets: with every key
+      // clamped and its block looked up lane by lane, a fifth of the kernel's
+      // VALU instructions were addresses.)
+      // the wave's side of the tile (its choice is scalar: one load either way)
+      const int64_t f16_stride_t = kw ? a.k_stride_t : a.v_stride_t;
+      const _Float16* f16 = (kw ? a.k_f16 + h * a.k_stride_h : a.v_f16 + h * a.v_stride_h) + k0 * f16_stride_t;
+      const uint32_t f16_pitch = (uint32_t)f16_stride_t * 2u;  // (launch_wide's caller bounds it)
+      const uint32_t f16_off = (uint32_t)(st >> 4) * f16_pitch + (uint32_t)(st & 15) * 16u;
+      const rsrc_t rc = kw ? kc : vc, rs = kw ? ks : vs;
+      // (K8V3's V: a group's three words and one neighbour, the next word or,
+      // for the key's last group, the word before)
+      const int gi = part >> 1;
+      const uint32_t lane_off = K8V3 && !kw ? (uint32_t)tt * (C::WORDS * 4) + (uint32_t)gi * 12u - (gi == 3 ? 4u : 0u)
+                                            : (uint32_t)tt * D + (uint32_t)part * 16u;
+      const uint32_t row_bytes = K8V3 && !kw ? C::WORDS * 4 : D;
+      char* const side = smem + (DENSE ? (kw ? (st >> 4) * C::KROW : C::KBYTES + (st >> 4) * C::VROW) + (st & 15) * 16
+                                       : (kw ? tt * C::KROW : C::KBYTES + tt * C::VROW) + part * 32);
+      // the block ids of kMaxSubBlocks - 2 blocks at a time (paged) in LDS
+      const int sub = DENSE ? k_hi - k_lo : (int)min((int64_t)(kMaxSubBlocks - 2) << bs_log2, (int64_t)(k_hi - k_lo));
+      for (int u0 = k_lo; u0 < k_hi; u0 += sub) {
+      const int u1 = min(k_hi, u0 + sub);
+      const int fb = u0 >> bs_log2, last_base = (u1 - 1) & ~(kTile - 1);
+      __syncthreads();  // previous users of bt_lds and the tile buffers are done
+      if constexpr (!DENSE) {
+        for (int i = tid; i <= ((u1 - 1) >> bs_log2) - fb; i += C::THREADS) bt_lds[i] = bt_row[fb + i];
         __syncthreads();
       }
+      // (tiles past the last one: the last one again)
+      auto block_id = [&](int base) -> int {
+        if constexpr (DENSE) return 0;
+        base = min(base, last_base);
+        return bt_lds[((bs_log2 >= 5 ? base : min(base + tt, u1 - 1)) >> bs_log2) - fb];
+      };
+      auto load_half = [&](HalfTile& R, int next) {
+        const int base = min(next, last_base);
+        if constexpr (DENSE) {  // keys past the sequence's last read as zeros
+          const rsrc_t r = make_rsrc(f16 + (int64_t)base * f16_stride_t,
+                                     (uint32_t)(min(nk - base, kTile) - 1) * f16_pitch + 2u * D);
+          R.d[0] = bload128(r, f16_off);
+          R.d[1] = bload128(r, f16_off + 16u * f16_pitch);
+        } else {
+          const int lim = min(u1 - 1 - base, kTile - 1);  // the tile's last key
+          const int key = min(tt, lim);
+          // one block: scalar offsets of its first row (rows past the last key
+          // are read too, and masked; not their scales); else a row per lane.
+          // (offsets are chosen and not loads: a choice of loads waits for those in flight)
+          const uint32_t bid = (uint32_t)__builtin_amdgcn_readfirstlane(R.bid);
+          uint32_t row = ((bid * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)base & bsm);
+          uint32_t off = lane_off, soff = (uint32_t)key * 4u;
+          if (bs_log2 < 5) {
+            row = 0;
+            const uint32_t lane_row =
+                (((uint32_t)R.bid * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)(base + key) & bsm);
+            off += (lane_row - (uint32_t)tt) * row_bytes;
+            soff = lane_row * 4u;
+          }
+          R.s = __builtin_bit_cast(float, bload32(rs, soff, row * 4u));
+          R.d[0] = bload128(rc, off, row * row_bytes);
+          R.bid = block_id(next + 2 * kTile);
+        }
+      };
+      auto store_half = [&](const HalfTile& R, int buf, int base) {
+        if constexpr (DENSE) {
+          *reinterpret_cast<u32x4_t*>(side + buf * C::BUF) = R.d[0];
+          *reinterpret_cast<u32x4_t*>(side + buf * C::BUF + 16 * (kw ? C::KROW : C::VROW)) = R.d[1];
+        } else {
+          if constexpr (!K8V3 && !FRESH) store16(side + buf * C::BUF, R.d[0]);
+          else if (kw) store_k(buf, base, tt, part, R.d[0]);
+          else store_v(buf, base, tt, st, K8V3 && gi == 3 ? u32x4_t{R.d[0].y, R.d[0].z, R.d[0].w, 0u} : R.d[0]);
+          if (part == 0) store_scale(buf, base, tt, kw, R.s);
+        }
+      };
+      auto half_barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const int ntiles = (u1 - u0 + kTile - 1) / kTile;
+      HalfTile r0, r1;
+      r0.bid = block_id(u0);
+      r1.bid = block_id(u0 + kTile);
+      load_half(r0, u0);
+      load_half(r1, u0 + kTile);
+      store_half(r0, 0, u0);
+      load_half(r0, u0 + 2 * kTile);
+      half_barrier();
+      if (!kw) half_barrier();
+      if constexpr (LIVE) {
+        qk(0);
+        qk_fresh(0, u0);
+      }
+      half_barrier();
+      // softmax of tile t (buffer `buf`), staging of tile t + 1 from R and
+      // the loads of tile t + 3; then PV(t) and QK(t + 1) (past the last
+      // tile: of stale keys, unused)
+      auto step = [&](HalfTile& R, int t, int buf) {
+        const int base = u0 + t * kTile;
+        store_half(R, buf ^ 1, base + kTile);
+        load_half(R, base + 3 * kTile);
+        half8_t va0[4];
+        if constexpr (LIVE) {
+          weights(buf, base, hides(base));
+#pragma unroll
+          for (int n = 0; n < 4; ++n) va0[n] = read_va(buf, 0, n);
+        }
+        half_barrier();
+        if constexpr (LIVE) {
+          half8_t va1[4], ka[8];
+          // PV and QK alternate, so that no MFMA follows the one whose result
+          // it adds to; LDS reads run 4 steps ahead (the scheduling barriers
+          // keep this order)
+          constexpr int NQ = DENSE ? 8 : 16;  // QK MFMAs: hi, or hi and lo
+          float16_t s = float16_t{};
+          auto qk_step = [&](int i) {
+            s = DENSE ? mfma32x32x16(ka[i], qhi[i], s) : mfma32x32x16(ka[i / 2], i & 1 ? qlo[i / 2] : qhi[i / 2], s);
+          };
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            // (K operand m is taken from step 4 + 2 m on, dense: 4 + m)
+            if (DENSE ? i < 8 : i % 2 == 0) ka[DENSE ? i : i / 2] = read_ka(buf ^ 1, DENSE ? i : i / 2);
+            if (i >= 4 && i < 8) va1[i - 4] = read_va(buf, 1, i - 4);
+            const u32x4_t w = i & 4 ? wl[i >> 3] : wh[i >> 3];
+            acc[i & 3] = mfma32x32x16(i < 8 ? va0[i & 3] : va1[i & 3], __builtin_bit_cast(half8_t, w), acc[i & 3]);
+            if (i >= 4 && i - 4 < NQ) qk_step(i - 4);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int i = 12; i < NQ; ++i) qk_step(i);
+          sc = s;
+          qk_fresh(buf ^ 1, base + kTile);
+        }
+        half_barrier();
+      };
+      int t = 0;  // (pairs in a loop of one block: a join inside it would wait for all loads)
+      for (; t + 1 < ntiles; t += 2) {
+        step(r1, t, 0);
+        step(r0, t + 1, 1);
+      }
+      if (t < ntiles) step(r1, t, 0);
+      if (kw) half_barrier();
+      }
+    } else {
+    for (int u0 = k_lo; u0 < k_hi; u0 += kSubKeys) {
+      const int u1 = min(k_hi, u0 + kSubKeys);
+      const int fb = u0 >> bs_log2;
+      const int nblk = ((u1 - 1) >> bs_log2) - fb + 1;
+      __syncthreads();  // previous users of bt_lds and the tile buffers are done
+      if constexpr (!DENSE)
+        for (int i = tid; i < nblk; i += C::THREADS) bt_lds[i] = bt_row[fb + i];
+      __syncthreads();
+
+      auto row_of = [&](int kk) -> uint32_t {
+        kk = min(kk, u1 - 1);
+        const uint32_t blk = (uint32_t)bt_lds[(kk >> bs_log2) - fb];
+        return ((blk * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)kk & bsm);
+      };
+      // dense: 512 16-byte fp16 K chunks and as many V chunks per tile, two
+      // each per thread
+      constexpr int NCH = DENSE ? 2 : 1;
+      struct TileRegs {
+        u32x4_t k[NCH], v[NCH];
+        float s;
+      };
+      // one 16-byte K chunk and one V chunk (K8V3: a half code group's three
+      // words) per thread, and the tile's 2 x 32 scales in threads 0..63
+      // (the cache rows of fresh drafts are loaded too, and not used)
+      auto load_tile = [&](TileRegs& R, int base) {
+        if constexpr (DENSE) {  // fp16 rows of keys base .. base + 31 (clamped to the last key)
+#pragma unroll
+          for (int i = 0; i < NCH; ++i) {
+            const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
+            const int64_t tok = k0 + min(base + tt, nk - 1);
+            R.k[i] = *reinterpret_cast<const u32x4_t*>(a.k_f16 + tok * a.k_stride_t + h * a.k_stride_h + part * 8);
+            R.v[i] = *reinterpret_cast<const u32x4_t*>(a.v_f16 + tok * a.v_stride_t + h * a.v_stride_h + part * 8);
+          }
+          return;
+        }
+        const int tt = tid >> 3, part = tid & 7;
+        const uint32_t row = row_of(base + tt);
+        R.k[0] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
+        if constexpr (K8V3) {
+          const u32x3_t w = bload96(vc, row * (uint32_t)(C::WORDS * 4) + (uint32_t)(part >> 1) * 12u);
+          R.v[0].x = w.x;
+          R.v[0].y = w.y;
+          R.v[0].z = w.z;
+        } else {
+          R.v[0] = bload128(vc, row * (uint32_t)D + (uint32_t)part * 16u);
+        }
+        // (two loads, each with one descriptor: a descriptor chosen per lane
+        // would be issued lane by lane)
+        if (tid < kTile) R.s = __builtin_bit_cast(float, bload32(ks, row_of(base + tid) * 4u));
+        else if (tid < 2 * kTile) R.s = __builtin_bit_cast(float, bload32(vs, row_of(base + tid - kTile) * 4u));
+      };
+      auto store_tile = [&](const TileRegs& R, int buf, int base) {
+        if constexpr (DENSE) {  // fp16 rows as they are
+          char* kb = smem + buf * C::BUF;
+          char* vb = kb + C::KBYTES;
+#pragma unroll
+          for (int i = 0; i < NCH; ++i) {
+            const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
+            *reinterpret_cast<u32x4_t*>(kb + tt * C::KROW + part * 16) = R.k[i];
+            *reinterpret_cast<u32x4_t*>(vb + tt * C::VROW + part * 16) = R.v[i];
+          }
+          return;
+        }
+        const int tt = tid >> 3, part = tid & 7;
+        store_k(buf, base, tt, part, R.k[0]);
+        store_v(buf, base, tt, tid, R.v[0]);
+        if (tid < 2 * kTile) store_scale(buf, base, tid & (kTile - 1), tid < kTile, R.s);
+      };
+      auto compute = [&](int buf, int base) {
+        if constexpr (LIVE) {
+          qk(buf);
+          qk_fresh(buf, base);
+          weights(buf, base, hides(base));
+          pv(buf);
+        }
+      };
+      const int ntiles = (u1 - u0 + kTile - 1) / kTile;
+      TileRegs ra, rb;
+      load_tile(ra, u0);
+      if (ntiles > 1) load_tile(rb, u0 + kTile);
+      store_tile(ra, 0, u0);
+      __syncthreads();
+      for (int t = 0; t < ntiles; t += 2) {  // (one exit: the accumulators keep their registers)
+        const int base = u0 + t * kTile;
+        if (t + 2 < ntiles) load_tile(ra, base + 2 * kTile);
+        compute(0, base);
+        if (t + 1 < ntiles) store_tile(rb, 1, base + kTile);
+        __syncthreads();
+        if (t + 1 < ntiles) {
+          if (t + 3 < ntiles) load_tile(rb, base + 3 * kTile);
+          compute(1, base + kTile);
+          if (t + 2 < ntiles) store_tile(ra, 0, base + 2 * kTile);
+          __syncthreads();
+        }
+      }
     }
-  }
+    }
   };
-  if (wave_live)
-    key_loop(std::true_type{});
-  else
-    key_loop(std::false_type{});
+  if (k_lo < k_hi) {
+    if (wave_live)
+      key_loop(std::true_type{});
+    else
+      key_loop(std::false_type{});
+  }
 
   const float l_tot = sum_x32(l_run);
   // ---- split: this wave's unnormalized rows to the partials ----
@@ -1988,8 +2188,11 @@ extern "C" int s8kv_attn_varlen_f16(const void* q, const void* k, const void* v,
   hipStream_t s = (hipStream_t)stream;
   // head_dim 128: the wide kernel (32 query rows per wave) when its vector
   // q loads (16 bytes) and output stores (8 bytes) are aligned
+  // (and K and V tiles keep 32-bit offsets)
+  auto tile_fits = [](int64_t stride_t) { return stride_t >= 0 && stride_t <= 1 << 25; };
   const bool wide = head_dim == 128 && (uintptr_t)q % 16 == 0 && q_stride_t % 8 == 0 && q_stride_h % 8 == 0 &&
-                    (uintptr_t)out % 8 == 0 && o_stride_t % 4 == 0 && o_stride_h % 4 == 0;
+                    (uintptr_t)out % 8 == 0 && o_stride_t % 4 == 0 && o_stride_h % 4 == 0 && tile_fits(k_stride_t) &&
+                    tile_fits(v_stride_t);
   if (wide)
     a.n_qblocks = (a.group * max_seqlen_q + verify::rows_per_wg(128, false, true, a.group * max_seqlen_q) - 1) /
                   verify::rows_per_wg(128, false, true, a.group * max_seqlen_q);

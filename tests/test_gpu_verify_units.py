@@ -17,20 +17,32 @@ from tests.kvgpu import CODEBOOK, alloc, append, assert_close, layer, t, to_np
 pytestmark = pytest.mark.gpu
 
 
-def _check(seed, kind, hq, hkv, d, bs, prefix, nq, what, query_lens=None, window=None):
+def _tree(rng, n):
+    """Ancestor bits of a random tree of n nodes."""
+    masks = np.zeros(n, np.uint64)
+    for i in range(n):
+        masks[i] = np.uint64(1) << np.uint64(i)
+        if i:
+            masks[i] |= masks[int(rng.integers(0, i))]
+    return masks.view(np.int64)
+
+
+def _check(seed, kind, hq, hkv, d, bs, prefix, nq, what, query_lens=None, window=None, tree=False):
     prefix = np.asarray(prefix)
     case = make_case(seed, len(prefix), hq, hkv, d, bs, prefix + nq, outlier_channels=2 if d >= 128 else 0)
     cache = alloc(kind, case.num_blocks, hkv, bs, d)
     append(kind, t(case.k), t(case.v), cache, t(case.slots))
     qv = np.random.default_rng(seed + 1).standard_normal((len(prefix), hq, nq, d)).astype(np.float16)
+    mask = np.stack([_tree(np.random.default_rng(seed + 2 + b), nq) for b in range(len(prefix))]) if tree else None
     fn = ops.attn_paged_verify if kind == "int8" else ops.attn_paged_verify_k8v3
     extra = () if kind == "int8" else (t(CODEBOOK),)
     out = fn(t(qv), *cache, *extra, t(case.block_table), t(prefix.astype(np.int32)), bs,
              query_lens=None if query_lens is None else t(np.asarray(query_lens, np.int32)),
-             max_context_len=int(case.lens.max()), scale=case.scale, window=window)
+             tree_mask=None if mask is None else t(mask), max_context_len=int(case.lens.max()), scale=case.scale,
+             window=window)
     torch.cuda.synchronize()
     ref = O.paged_verify(qv, layer(kind, tuple(to_np(x) for x in cache)), case.block_table, prefix, case.scale,
-                         query_lens=query_lens, window=window)
+                         query_lens=query_lens, window=window, tree_mask=mask)
     got = to_np(out.float())
     for b, n in enumerate([] if query_lens is None else query_lens):
         assert not got[b, :, n:].any(), f"{what}: row {b}, outputs past its {n} queries"
@@ -72,6 +84,19 @@ def test_equal_splits_of_ragged_rows(kind, d, window):
     prefix, nq = [2600, 0, 511, 512, 513, 1023, 1024, 31, 33], 5
     lens = [5, 5, 1, 5, 0, 2, 5, 5, 3]
     _check(80 + d, kind, 8, 2, d, 32, prefix, nq, f"{kind} D={d} window={window}", query_lens=lens, window=window)
+
+
+@pytest.mark.parametrize("kind", ["int8", "k8v3"])
+@pytest.mark.parametrize("bs,nq,tree", [(4, 40, False), (8, 64, True), (32, 64, True), (256, 33, False)])
+@pytest.mark.parametrize("window", [None, 40])
+def test_more_than_128_rows(kind, bs, nq, tree, window):
+    """Rows enough for 8-wave workgroups (G 4): prefixes that start the drafts
+    at every kind of place in a 32-key tile, one to three tiles in all, odd and
+    even tile counts, more blocks than are looked up at a time (bs 4, 2,047
+    keys and up), blocks smaller than a tile, and waves without a live row."""
+    prefix = [0, 1, 31, 32, 33, 64, 95, 2047 + 5 * bs, 700]
+    _check(300 + bs + nq, kind, 8, 2, 128, bs, prefix, nq, f"{kind} bs={bs} nq={nq} tree={tree} window={window}",
+           query_lens=[nq, nq, 1, nq - 1, nq, 9, nq, nq, 0], window=window, tree=tree)
 
 
 def test_workspace_counts_the_split():
