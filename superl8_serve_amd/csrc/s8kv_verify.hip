@@ -819,12 +819,12 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
 }
 
 // ---------------------------------------------------------------------------
-// Wide verify (head_dim 128, paged int8 or K8V3 cache): 32 query rows per wave
+// Wide verify (head_dim 128 and 256; paged int8 or K8V3 cache, or dense): 32 query rows per wave
 // on v_mfma_f32_32x32x16_f16, so every K and V operand a wave reads from LDS
 // feeds twice the MFMAs of a 16-row wave.  Lane (j = lane % 32, hf = lane /
-// 32) holds query row j of its wave:
-//   QK  : S^T[key][row] with A = K rows from LDS (key lane % 32, dims 64 hf ..
-//         64 hf + 63, 8 per MFMA), B = the rotated, pre-scaled q of row j over
+// 32) holds query row j of its wave (head_dim D):
+//   QK  : S^T[key][row] with A = K rows from LDS (key lane % 32, dims D / 2 hf
+//         .., 8 per MFMA), B = the rotated, pre-scaled q of row j over
 //         the same dims as fp16 hi + lo; lane l's result register r is key
 //         8 (r / 4) + 4 hf + r % 4 of row j, so the softmax state of a row
 //         lives in one lane pair (lane, lane ^ 32).
@@ -857,28 +857,32 @@ __device__ __forceinline__ void split_pair(float w0, float w1, uint32_t& hi, uin
   lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(l0, l1));
 }
 
-template <bool K8V3, bool EIGHT>
+template <int D, bool K8V3, bool EIGHT>
 struct WideCfg {
-  static constexpr int D = 128;
+  static_assert(D == 128 || (D == 256 && !EIGHT), "head_dim 256: 4 waves");
   // EIGHT (calls with more than 128 query rows per sequence and KV head):
   // 8 waves (256 rows) per workgroup, one workgroup per CU, so twice the rows
   // share each tile's staging (K8V3: code expansion); else 4 waves, two per CU
   static constexpr int WAVES = EIGHT ? 8 : 4;
-  static constexpr int WG_PER_CU = 8 / WAVES;
+  // head_dim 256: one wave per SIMD, whose 512 registers hold the row group's
+  // accumulators and q hi + lo (128 each)
+  static constexpr int WG_PER_CU = D == 256 ? 1 : 8 / WAVES;
   static constexpr int THREADS = 64 * WAVES;
   static constexpr int ROWS = 32 * WAVES;  // query rows per workgroup
   static constexpr int KROW = 2 * D + 16;  // LDS pitch of an fp16 K row (8 consecutive rows: distinct 16-byte slots)
   static constexpr int VROW = 2 * D + 32;  // LDS pitch of an fp16 V row (4 rows of a transpose read: distinct banks)
   static constexpr int KBYTES = kTile * KROW;
   static constexpr int VBYTES = kTile * VROW;
-  static constexpr int SBYTES = 2 * kTile * 4;  // k_scale, then the V scale (int8) or block norm (K8V3) per key
+  static constexpr int NB = K8V3 ? D / 128 : 1;  // V scales per key: the int8 row scale, or K8V3 block norms
+  static constexpr int SBYTES = (1 + NB) * kTile * 4;  // k_scale, then the V scales of each block
   static constexpr int BUF = KBYTES + VBYTES + SBYTES;
-  static constexpr int CHUNKS = kTile * D / 16;  // 16-byte int8 chunks per K (or V) tile: one per thread
-  static_assert(CHUNKS == 256, "one K chunk per thread of the first 256 (and one V chunk per thread of the last)");
+  static constexpr int PARTS = D / 16;   // 16-byte int8 chunks of a key's K (or V); K8V3: half code groups
+  static constexpr int NCH = EIGHT ? 1 : kTile * PARTS / THREADS;  // of a tile, per thread (EIGHT: K, or V)
   static constexpr int NG = D / 32;      // K8V3: 32-value code groups per key
   static constexpr int WORDS = 3 * NG;   // K8V3: packed words per key
-  static constexpr int VJOBS = 2 * kTile * NG;  // K8V3: two threads per code group (16 values each)
-  static_assert(VJOBS == 256, "one K8V3 expansion job per thread of the last 256");
+  static constexpr int HALF = D / 2;     // dims a lane holds of q and takes of a K row
+  static constexpr int NM = D / 16;      // QK MFMAs (of hi or lo)
+  static constexpr int NT = D / 32;      // 32-dim tiles of the output
   static constexpr int SMEM = 2 * BUF + kMaxSubBlocks * 4;
   // window verify with fresh drafts: the low fp16 part of the drafts' K per buffer
   static constexpr int KLO_OFF = (SMEM + 15) / 16 * 16;
@@ -892,13 +896,14 @@ struct WideCfg {
 // every row sees the last `window` prefix keys and the drafts, keys j >=
 // prefix - window, the drafts' K / V from the cache or (FRESH, a.kd set) from
 // the fresh fp32 K (rotated) and fp16 V rows of the drafts.
-template <bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false, bool EIGHT = false>
-__global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIGHT>::WG_PER_CU)) void verify_wide_kernel(
+template <int D, bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false, bool EIGHT = false>
+__global__
+__launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::WG_PER_CU)) void verify_wide_kernel(
     VerifyArgs a) {
   static_assert(!(DENSE && K8V3), "dense inputs: fp16 K / V");
   static_assert(!FRESH || (WIN && !DENSE), "fresh drafts: a paged window verify");
-  using C = WideCfg<K8V3, EIGHT>;
-  constexpr int D = C::D;
+  using C = WideCfg<D, K8V3, EIGHT>;
+  constexpr int NM = C::NM, NT = C::NT, NB = C::NB, PARTS = C::PARTS, HALF = C::HALF;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int* bt_lds = reinterpret_cast<int*>(smem + 2 * C::BUF);
 
@@ -950,28 +955,28 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   const bool row_live = pos < nq;
   const uint64_t tmask = (tree && row_live) ? (uint64_t)a.tree_mask[(int64_t)b * a.max_queries + pos] : 0ull;
 
-  // ---- q: rotate (FWHT over dims 64 hf .. 64 hf + 63 in-lane, then across
+  // ---- q: rotate (FWHT over dims D / 2 hf .. in-lane, then across
   // the lane pair), pre-scale, split into fp16 hi + lo; dense: the fp16 input ----
-  half8_t qhi[8], qlo[DENSE ? 1 : 8];
+  half8_t qhi[NM], qlo[DENSE ? 1 : NM];
   if constexpr (DENSE) {
     const _Float16* qp = a.q + (int64_t)q0 * a.q_stride_s + (int64_t)head * a.q_stride_h +
-                         (int64_t)(row_live ? pos : 0) * a.q_stride_s + hf * 64;
+                         (int64_t)(row_live ? pos : 0) * a.q_stride_s + hf * HALF;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) qhi[m] = row_live ? *reinterpret_cast<const half8_t*>(qp + 8 * m) : half8_t{};
+    for (int m = 0; m < NM; ++m) qhi[m] = row_live ? *reinterpret_cast<const half8_t*>(qp + 8 * m) : half8_t{};
   } else {
-    float x[64];
+    float x[HALF];
     const _Float16* qp = a.q + (int64_t)b * a.q_stride_b + (int64_t)head * a.q_stride_h +
-                         (int64_t)(row_live ? pos : 0) * a.q_stride_s + hf * 64;
+                         (int64_t)(row_live ? pos : 0) * a.q_stride_s + hf * HALF;
 #pragma unroll
-    for (int i = 0; i < 64; i += 8) {
+    for (int i = 0; i < HALF; i += 8) {
       const half8_t v = *reinterpret_cast<const half8_t*>(qp + i);
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[i + e] = row_live ? (float)v[e] : 0.0f;
     }
 #pragma unroll
-    for (int hs = 1; hs < 64; hs <<= 1) {
+    for (int hs = 1; hs < HALF; hs <<= 1) {
 #pragma unroll
-      for (int i = 0; i < 64; ++i) {
+      for (int i = 0; i < HALF; ++i) {
         if ((i & hs) == 0) {
           const float x0 = x[i], x1 = x[i + hs];
           x[i] = x0 + x1;
@@ -980,9 +985,9 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
       }
     }
 #pragma unroll
-    for (int i = 0; i < 64; ++i) x[i] = butterfly_x32(x[i], lane);
+    for (int i = 0; i < HALF; ++i) x[i] = butterfly_x32(x[i], lane);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
+    for (int m = 0; m < NM; ++m) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         // (materialized: hi and lo must both come from this one fp32 value)
@@ -995,9 +1000,9 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   }
 
   float m_ref = kMaxInit, l_run = 0.0f;
-  float16_t acc[4];
+  float16_t acc[NT];
 #pragma unroll
-  for (int n = 0; n < 4; ++n) acc[n] = float16_t{};
+  for (int n = 0; n < NT; ++n) acc[n] = float16_t{};
   WeightShift ws(kMaxSlack);
   if constexpr (DENSE) ws.raise(1.0f, kMaxSlack);  // fp16 K / V: every V scale is 1
 
@@ -1074,7 +1079,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
     char* vb = smem + buf * C::BUF + C::KBYTES + tt * C::VROW;
     const int di = fresh_draft(base, tt);
     if (di >= 0) {
-      const int part = vt & 7;
+      const int part = vt % PARTS;
       const half8_t* vp = reinterpret_cast<const half8_t*>(
           a.vd + (int64_t)b * a.vd_stride_b + (int64_t)di * a.vd_stride_s + (int64_t)h * a.vd_stride_h + part * 16);
       *reinterpret_cast<half8_t*>(vb + part * 32) = vp[0];
@@ -1082,9 +1087,9 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
       return;
     }
     if constexpr (!K8V3) {
-      store16(vb + (vt & 7) * 32, d);
+      store16(vb + (vt % PARTS) * 32, d);
     } else {  // 16 codes of one group -> fp16 codebook entries
-      const int gi = (vt >> 1) & 3, sh = (vt & 1) * 16;
+      const int gi = (vt >> 1) % C::NG, sh = (vt & 1) * 16;
       const uint32_t w0 = d.x >> sh, w1 = d.y >> sh, w2 = d.z >> sh;
       char* dst = vb + gi * 64 + sh * 2;
 #pragma unroll
@@ -1104,34 +1109,38 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   // key, exp2(-inf) * scale, is then 0 whatever was stored there (clamped
   // here, where the load is consumed, not where it is issued); a fresh
   // draft's K and V scales are 1
-  auto store_scale = [&](int buf, int base, int tt, bool k_side, float v) {
+  auto store_scale = [&](int buf, int base, int tt, int side, float v) {  // side 0: K, 1 + n: V block n
     float* sb = reinterpret_cast<float*>(smem + buf * C::BUF + C::KBYTES + C::VBYTES);
-    sb[k_side ? tt : kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : k_side ? v : fminf(v, 0x1p100f);
+    const bool k_side = side == 0;
+    sb[side * kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : k_side ? v : fminf(v, 0x1p100f);
   };
 
   // ---- one 32-key tile from LDS buffer `buf`: scores, weights, PV ----
   float16_t sc;
-  u32x4_t wh[2], wl[2];  // weights of keys 16t .. 16t + 15 as fp16 hi + lo
+  u32x4_t wh[NB][2], wl[NB][2];  // weights (per V block) of keys 16t .. 16t + 15 as fp16 hi + lo
   auto read_ka = [&](int buf, int m) -> half8_t {
-    return *reinterpret_cast<const half8_t*>(smem + buf * C::BUF + j * C::KROW + hf * 128 + 16 * m);
+    return *reinterpret_cast<const half8_t*>(smem + buf * C::BUF + j * C::KROW + hf * D + 16 * m);
   };
   auto qk = [&](int buf) {
-    half8_t ka[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) ka[m] = read_ka(buf, m);
     sc = float16_t{};
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      sc = mfma32x32x16(ka[m], qhi[m], sc);
-      if constexpr (!DENSE) sc = mfma32x32x16(ka[m], qlo[m], sc);
+    for (int m0 = 0; m0 < NM; m0 += 8) {
+      half8_t ka[8];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) ka[m] = read_ka(buf, m0 + m);
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        sc = mfma32x32x16(ka[m], qhi[m0 + m], sc);
+        if constexpr (!DENSE) sc = mfma32x32x16(ka[m], qlo[m0 + m], sc);
+      }
     }
   };
   auto qk_fresh = [&](int buf, int base) {
     if constexpr (FRESH) {  // fresh draft keys: K = hi + lo
       if (fresh_tile(base)) {
-        const char* lrow = smem + C::KLO_OFF + buf * C::KBYTES + j * C::KROW + hf * 128;
+        const char* lrow = smem + C::KLO_OFF + buf * C::KBYTES + j * C::KROW + hf * D;
 #pragma unroll
-        for (int m = 0; m < 8; ++m) sc = mfma32x32x16(*reinterpret_cast<const half8_t*>(lrow + 16 * m), qhi[m], sc);
+        for (int m = 0; m < NM; ++m) sc = mfma32x32x16(*reinterpret_cast<const half8_t*>(lrow + 16 * m), qhi[m], sc);
       }
     }
   };
@@ -1177,7 +1186,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
     // V-scale bound test: lane l checks the V scale of key l % 32 (paged
     // window: not of the keys below it, which may hold anything)
     float vp = 0.0f;
-    if constexpr (!DENSE) vp = sb[kTile + j];
+    if constexpr (!DENSE) vp = NB == 2 ? fmaxf(sb[kTile + j], sb[2 * kTile + j]) : sb[kTile + j];
     if constexpr (WIN && !DENSE) vp = base + j >= lo_key ? vp : 0.0f;
     if (__builtin_amdgcn_ballot_w64(my > ws.thr() || vp > ws.vbound()) != 0) {
       // rare: a V scale above the bound lowers the weight shift (by d, a
@@ -1201,7 +1210,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
       const float alpha = __builtin_amdgcn_exp2f(m_ref - m_new) * __builtin_ldexpf(1.0f, d);
       l_run *= alpha;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) acc[n] *= alpha;  // (plain VALU: its MFMA hazards are the compiler's)
+      for (int n = 0; n < NT; ++n) acc[n] *= alpha;  // (plain VALU: its MFMA hazards are the compiler's)
       m_ref = m_new;
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) y[rr] = y[rr] != kNegInf ? __builtin_fmaf(sc[rr], kscale(rr), -m_new) : kNegInf;
@@ -1212,28 +1221,34 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
       // hi + lo (hi: the top 11 significant bits, exact in fp16 over its
       // normal range; lo: the rest); hidden keys weigh 0 whatever their
       // scale (inf and NaN included)
-      float4_t vs0{}, vs1{};
-      if constexpr (!DENSE) {
-        vs0 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 4 * hf);
-        vs1 = *reinterpret_cast<const float4_t*>(sb + kTile + 16 * t + 8 + 4 * hf);
+      float ev[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        ev[e] = __builtin_amdgcn_exp2f(y[8 * t + e]);  // 0 for hidden keys
+        l_run += ev[e];
       }
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        float w[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int rr = 8 * t + e + u;
-          const float ev = __builtin_amdgcn_exp2f(y[rr]);  // 0 for hidden keys
-          l_run += ev;
-          // (finite scales: 0 for hidden keys; dense: ev itself, which
-          // split_pair's rounding reads before its asm does)
-          if constexpr (DENSE) w[u] = ev;
-          else w[u] = ev * (e + u < 4 ? vs0[e + u] : vs1[e + u - 4]);
+      for (int nb = 0; nb < NB; ++nb) {
+        float4_t vs0{}, vs1{};
+        if constexpr (!DENSE) {
+          vs0 = *reinterpret_cast<const float4_t*>(sb + (1 + nb) * kTile + 16 * t + 4 * hf);
+          vs1 = *reinterpret_cast<const float4_t*>(sb + (1 + nb) * kTile + 16 * t + 8 + 4 * hf);
         }
-        uint32_t hw, lw;
-        split_pair(w[0], w[1], hw, lw);
-        wh[t][e / 2] = hw;
-        wl[t][e / 2] = lw;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          float w[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            // (finite scales: 0 for hidden keys; dense: ev itself, which
+            // split_pair's rounding reads before its asm does)
+            if constexpr (DENSE) w[u] = ev[e + u];
+            else w[u] = ev[e + u] * (e + u < 4 ? vs0[e + u] : vs1[e + u - 4]);
+          }
+          uint32_t hw, lw;
+          split_pair(w[0], w[1], hw, lw);
+          wh[nb][t][e / 2] = hw;
+          wl[nb][t][e / 2] = lw;
+        }
       }
     }
   };
@@ -1252,12 +1267,12 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   auto pv = [&](int buf) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const half8_t pbh = __builtin_bit_cast(half8_t, wh[t]), pbl = __builtin_bit_cast(half8_t, wl[t]);
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < NT; ++n) {
+        const int nb = n * NB / NT;
         const half8_t va = read_va(buf, t, n);
-        acc[n] = mfma32x32x16(va, pbh, acc[n]);
-        acc[n] = mfma32x32x16(va, pbl, acc[n]);
+        acc[n] = mfma32x32x16(va, __builtin_bit_cast(half8_t, wh[nb][t]), acc[n]);
+        acc[n] = mfma32x32x16(va, __builtin_bit_cast(half8_t, wl[nb][t]), acc[n]);
       }
     }
   };
@@ -1370,7 +1385,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
           if constexpr (!K8V3 && !FRESH) store16(side + buf * C::BUF, R.d[0]);
           else if (kw) store_k(buf, base, tt, part, R.d[0]);
           else store_v(buf, base, tt, st, K8V3 && gi == 3 ? u32x4_t{R.d[0].y, R.d[0].z, R.d[0].w, 0u} : R.d[0]);
-          if (part == 0) store_scale(buf, base, tt, kw, R.s);
+          if (part == 0) store_scale(buf, base, tt, kw ? 0 : 1, R.s);
         }
       };
       auto half_barrier = [&]() {
@@ -1422,7 +1437,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
             // (K operand m is taken from step 4 + 2 m on, dense: 4 + m)
             if (DENSE ? i < 8 : i % 2 == 0) ka[DENSE ? i : i / 2] = read_ka(buf ^ 1, DENSE ? i : i / 2);
             if (i >= 4 && i < 8) va1[i - 4] = read_va(buf, 1, i - 4);
-            const u32x4_t w = i & 4 ? wl[i >> 3] : wh[i >> 3];
+            const u32x4_t w = i & 4 ? wl[0][i >> 3] : wh[0][i >> 3];
             acc[i & 3] = mfma32x32x16(i < 8 ? va0[i & 3] : va1[i & 3], __builtin_bit_cast(half8_t, w), acc[i & 3]);
             if (i >= 4 && i - 4 < NQ) qk_step(i - 4);
             __builtin_amdgcn_sched_barrier(0);
@@ -1457,59 +1472,64 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
         const uint32_t blk = (uint32_t)bt_lds[(kk >> bs_log2) - fb];
         return ((blk * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)kk & bsm);
       };
-      // dense: 512 16-byte fp16 K chunks and as many V chunks per tile, two
-      // each per thread
-      constexpr int NCH = DENSE ? 2 : 1;
+      // 16-byte chunks of the tile's K and V per thread: int8 (K8V3 V: a half
+      // code group's three words), or fp16
+      constexpr int NCH = DENSE ? 2 * C::NCH : C::NCH;
       struct TileRegs {
         u32x4_t k[NCH], v[NCH];
         float s;
       };
-      // one 16-byte K chunk and one V chunk (K8V3: a half code group's three
-      // words) per thread, and the tile's 2 x 32 scales in threads 0..63
-      // (the cache rows of fresh drafts are loaded too, and not used)
+      // (and the tile's scales in threads 0..; the cache rows of fresh drafts
+      // are loaded too, and not used)
       auto load_tile = [&](TileRegs& R, int base) {
         if constexpr (DENSE) {  // fp16 rows of keys base .. base + 31 (clamped to the last key)
 #pragma unroll
           for (int i = 0; i < NCH; ++i) {
-            const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
+            const int ch = tid + i * C::THREADS, tt = ch / (2 * PARTS), part = ch % (2 * PARTS);
             const int64_t tok = k0 + min(base + tt, nk - 1);
             R.k[i] = *reinterpret_cast<const u32x4_t*>(a.k_f16 + tok * a.k_stride_t + h * a.k_stride_h + part * 8);
             R.v[i] = *reinterpret_cast<const u32x4_t*>(a.v_f16 + tok * a.v_stride_t + h * a.v_stride_h + part * 8);
           }
           return;
         }
-        const int tt = tid >> 3, part = tid & 7;
-        const uint32_t row = row_of(base + tt);
-        R.k[0] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
-        if constexpr (K8V3) {
-          const u32x3_t w = bload96(vc, row * (uint32_t)(C::WORDS * 4) + (uint32_t)(part >> 1) * 12u);
-          R.v[0].x = w.x;
-          R.v[0].y = w.y;
-          R.v[0].z = w.z;
-        } else {
-          R.v[0] = bload128(vc, row * (uint32_t)D + (uint32_t)part * 16u);
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+          const int ch = tid + i * C::THREADS, tt = ch / PARTS, part = ch % PARTS;
+          const uint32_t row = row_of(base + tt);
+          R.k[i] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
+          if constexpr (K8V3) {
+            const u32x3_t w = bload96(vc, row * (uint32_t)(C::WORDS * 4) + (uint32_t)(part >> 1) * 12u);
+            R.v[i].x = w.x;
+            R.v[i].y = w.y;
+            R.v[i].z = w.z;
+          } else {
+            R.v[i] = bload128(vc, row * (uint32_t)D + (uint32_t)part * 16u);
+          }
         }
         // (two loads, each with one descriptor: a descriptor chosen per lane
         // would be issued lane by lane)
-        if (tid < kTile) R.s = __builtin_bit_cast(float, bload32(ks, row_of(base + tid) * 4u));
-        else if (tid < 2 * kTile) R.s = __builtin_bit_cast(float, bload32(vs, row_of(base + tid - kTile) * 4u));
+        const int tk = tid & (kTile - 1);
+        if (tid < kTile) R.s = __builtin_bit_cast(float, bload32(ks, row_of(base + tk) * 4u));
+        else if (tid < (1 + NB) * kTile)
+          R.s = __builtin_bit_cast(float, bload32(vs, (row_of(base + tk) * NB + (tid / kTile - 1)) * 4u));
       };
       auto store_tile = [&](const TileRegs& R, int buf, int base) {
-        if constexpr (DENSE) {  // fp16 rows as they are
-          char* kb = smem + buf * C::BUF;
-          char* vb = kb + C::KBYTES;
 #pragma unroll
-          for (int i = 0; i < NCH; ++i) {
-            const int ch = tid + i * C::THREADS, tt = ch >> 4, part = ch & 15;
+        for (int i = 0; i < NCH; ++i) {
+          const int ch = tid + i * C::THREADS;
+          if constexpr (DENSE) {  // fp16 rows as they are
+            char* kb = smem + buf * C::BUF;
+            const int tt = ch / (2 * PARTS), part = ch % (2 * PARTS);
             *reinterpret_cast<u32x4_t*>(kb + tt * C::KROW + part * 16) = R.k[i];
-            *reinterpret_cast<u32x4_t*>(vb + tt * C::VROW + part * 16) = R.v[i];
+            *reinterpret_cast<u32x4_t*>(kb + C::KBYTES + tt * C::VROW + part * 16) = R.v[i];
+          } else {
+            const int tt = ch / PARTS;
+            store_k(buf, base, tt, ch % PARTS, R.k[i]);
+            store_v(buf, base, tt, ch, R.v[i]);
           }
-          return;
         }
-        const int tt = tid >> 3, part = tid & 7;
-        store_k(buf, base, tt, part, R.k[0]);
-        store_v(buf, base, tt, tid, R.v[0]);
-        if (tid < 2 * kTile) store_scale(buf, base, tid & (kTile - 1), tid < kTile, R.s);
+        if constexpr (!DENSE)
+          if (tid < (1 + NB) * kTile) store_scale(buf, base, tid & (kTile - 1), tid / kTile, R.s);
       };
       auto compute = [&](int buf, int base) {
         if constexpr (LIVE) {
@@ -1555,7 +1575,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
     const int rl = wave * 32 + j;
     float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * a.part_rows + rl) * (D + 4);
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < NT; ++n) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<float4_t*>(pr + 32 * n + 8 * q + 4 * hf) =
@@ -1574,7 +1594,7 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
     _Float16* op = DENSE ? a.out + (int64_t)(q0 + pos) * a.o_stride_t + (int64_t)head * a.o_stride_h
                          : a.out + (((int64_t)b * a.num_q_heads + head) * a.max_queries + pos) * D;
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < NT; ++n) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         half4_t o;
@@ -1586,22 +1606,25 @@ __global__ __launch_bounds__((WideCfg<K8V3, EIGHT>::THREADS), (WideCfg<K8V3, EIG
   }
 }
 
-// The wide kernel serves the paged head_dim-128 calls whose tensors fit
-// 32-bit offsets (no per-tile descriptor rebasing), with or without a window.
+// The wide kernel serves the paged head_dim-128 and -256 calls whose tensors
+// fit 32-bit offsets (no per-tile descriptor rebasing), with or without a
+// window.  Head_dim 256 in the 16-row kernel: its accumulators and q hi + lo
+// left no registers at two waves per SIMD (over 400 bytes of spills a lane);
+// one sequence of 1,999 queries over 6,007 keys, 4 KV heads, group 4: 2,200
+// -> 809 us; 7 dense prompts of up to 2,248, 8 heads over 4: 992 -> 244.
 // Query rows per workgroup at this head_dim and layout (Cfg<D, K8V3>::ROWS,
 // or WideCfg::ROWS for the wide kernel), and the workgroups a CU keeps
 // resident (the kernels' launch bounds).
-static bool use_wide(int head_dim, bool big) { return head_dim == 128 && !big; }
+static bool use_wide(int head_dim, bool big) { return (head_dim == 128 || head_dim == 256) && !big; }
 // rows: query rows per (sequence, KV head) -- group x max_queries; the wide
-// kernel takes 8-wave workgroups when they exceed one 4-wave block
-static bool wide_eight(int rows) { return rows > WideCfg<false, false>::ROWS; }
+// kernel takes 8-wave workgroups at head_dim 128 when they exceed one 4-wave block
+static bool wide_eight(int head_dim, int rows) { return head_dim == 128 && rows > WideCfg<128, false, false>::ROWS; }
 static int rows_per_wg(int head_dim, bool k8v3, bool wide, int rows) {
-  if (wide) return wide_eight(rows) ? WideCfg<false, true>::ROWS : WideCfg<false, false>::ROWS;
+  if (wide) return wide_eight(head_dim, rows) ? WideCfg<128, false, true>::ROWS : WideCfg<128, false, false>::ROWS;
   return 16 * (k8v3 ? 8 : 4) * (head_dim <= 64 ? 2 : 1);
 }
-static int wg_per_cu(bool k8v3, bool wide, int rows) {
-  return wide ? (wide_eight(rows) ? WideCfg<false, true>::WG_PER_CU : WideCfg<false, false>::WG_PER_CU)
-              : (k8v3 ? 1 : 2);
+static int wg_per_cu(int head_dim, bool k8v3, bool wide, int rows) {
+  return wide ? (wide_eight(head_dim, rows) || head_dim == 256 ? 1 : 2) : (k8v3 ? 1 : 2);
 }
 
 // Combine of a split verify: one thread per (row, 4 dims) of a (sequence,
@@ -1733,18 +1756,20 @@ template <int D, bool K8V3, bool WIN = false, bool DENSE = false>
 static int launch(VerifyArgs& a, hipStream_t stream) {
   if constexpr (DENSE)
     return launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
+  else if constexpr (D >= 128)  // (the wide kernel serves the others)
+    return launch_impl<D, K8V3, WIN, DENSE, true>(a, stream);
   else
     return a.big ? launch_impl<D, K8V3, WIN, DENSE, true>(a, stream)
                  : launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
 }
 
-template <bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT>
+template <int D, bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT>
 static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
-  using C = WideCfg<K8V3, EIGHT>;
+  using C = WideCfg<D, K8V3, EIGHT>;
   constexpr int smem = FRESH ? C::SMEM_WIN : C::SMEM;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_wide_kernel<K8V3, DENSE, WIN, FRESH, EIGHT>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
       set_error("s8kv_verify: cannot set the dynamic LDS size");
       return S8KV_ERR_LAUNCH;
@@ -1757,12 +1782,12 @@ static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
     set_error("s8kv_verify: grid too large");
     return S8KV_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((verify_wide_kernel<K8V3, DENSE, WIN, FRESH, EIGHT>), dim3((unsigned)grid), dim3(C::THREADS), smem,
+  hipLaunchKernelGGL((verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT>), dim3((unsigned)grid), dim3(C::THREADS), smem,
                      stream, a);
   if (a.splits > 1) {
     const int rc = check_launch("s8kv_verify");
     if (rc != S8KV_OK) return rc;
-    return launch_combine<C::D, C::ROWS>(a, (int64_t)P * a.n_qblocks, stream);
+    return launch_combine<D, C::ROWS>(a, (int64_t)P * a.n_qblocks, stream);
   }
   return check_launch("s8kv_verify");
 }
@@ -1772,9 +1797,10 @@ static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
 // idle: 13 % slower); the host sized n_qblocks and the split by the same
 // rule (rows_per_wg, wg_per_cu)
 template <bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false>
-static int launch_wide(VerifyArgs& a, hipStream_t stream) {
-  if (wide_eight(a.group * a.max_queries)) return launch_wide_impl<K8V3, DENSE, WIN, FRESH, true>(a, stream);
-  return launch_wide_impl<K8V3, DENSE, WIN, FRESH, false>(a, stream);
+static int launch_wide(VerifyArgs& a, int head_dim, hipStream_t stream) {
+  if (head_dim == 256) return launch_wide_impl<256, K8V3, DENSE, WIN, FRESH, false>(a, stream);
+  if (wide_eight(head_dim, a.group * a.max_queries)) return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, true>(a, stream);
+  return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, false>(a, stream);
 }
 
 }  // namespace verify
@@ -1815,10 +1841,10 @@ constexpr int kBalanceRounds = 8;
 constexpr int kMaxSplitKeys = 1 << 20;
 constexpr int kMaxSplits = 1024;
 static std::atomic<int> g_verify_splits{0};  // 0: planned per call
-static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int keys, bool k8v3, bool wide, int rows,
-                              int rows_wg) {
+static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int keys, int head_dim, bool k8v3, bool wide,
+                              int rows, int rows_wg) {
   const int64_t natural = (int64_t)batch * num_kv_heads * n_qblocks;
-  const int64_t resident = (int64_t)verify::wg_per_cu(k8v3, wide, rows) * device_cus();
+  const int64_t resident = (int64_t)verify::wg_per_cu(head_dim, k8v3, wide, rows) * device_cus();
   int64_t s = natural < resident ? (resident + natural - 1) / natural : 1;
   s = std::min<int64_t>(s, std::max(1, keys / kMinSplitKeys));
   if (batch > 1) {
@@ -1847,13 +1873,13 @@ extern "C" int64_t s8kv_verify_workspace_size(int batch, int num_q_heads, int nu
   int64_t need = 0;
   for (const bool k8v3 : {false, true}) {
     for (const bool wide : {false, true}) {
-      if (wide && head_dim != 128) continue;
+      if (wide && head_dim == 64) continue;
       const int rows = num_q_heads / num_kv_heads * max_queries;
       const int rows_wg = verify::rows_per_wg(head_dim, k8v3, wide, rows);
       const int n_qblocks = (rows + rows_wg - 1) / rows_wg;
       need = std::max(need, verify_part_bytes(batch, num_kv_heads, n_qblocks, head_dim,
                                               verify_plan_splits(batch, num_kv_heads, n_qblocks, max_context_len,
-                                                                 k8v3, wide, rows, rows_wg),
+                                                                 head_dim, k8v3, wide, rows, rows_wg),
                                               rows, rows_wg));
     }
   }
@@ -1873,7 +1899,7 @@ static int verify_use_workspace(verify::VerifyArgs& a, int head_dim, bool k8v3, 
                                 : a.max_context_len;
   const int rows = a.group * a.max_queries;
   const int rows_wg = verify::rows_per_wg(head_dim, k8v3, wide, rows);
-  const int s = verify_plan_splits(a.batch, a.num_kv_heads, a.n_qblocks, keys, k8v3, wide, rows, rows_wg);
+  const int s = verify_plan_splits(a.batch, a.num_kv_heads, a.n_qblocks, keys, head_dim, k8v3, wide, rows, rows_wg);
   const int64_t need = verify_part_bytes(a.batch, a.num_kv_heads, a.n_qblocks, head_dim, s, rows, rows_wg);
   const bool fits = workspace != nullptr && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
   if (s > 1 && fits) {
@@ -1995,8 +2021,8 @@ static int verify_int8_impl(const void* q, int batch, int num_q_heads, int num_k
   a.vs_bytes = a.ks_bytes;
   hipStream_t s = (hipStream_t)stream;
   if (wide) {
-    if (a.kd != nullptr) return verify::launch_wide<false, false, true, true>(a, s);
-    return a.window > 0 ? verify::launch_wide<false, false, true>(a, s) : verify::launch_wide<false>(a, s);
+    if (a.kd != nullptr) return verify::launch_wide<false, false, true, true>(a, head_dim, s);
+    return a.window > 0 ? verify::launch_wide<false, false, true>(a, head_dim, s) : verify::launch_wide<false>(a, head_dim, s);
   }
   if (a.window > 0) {
     switch (head_dim) {
@@ -2095,8 +2121,8 @@ static int verify_k8v3_impl(const void* q, int batch, int num_q_heads, int num_k
   a.vs_bytes = cap_u32(a.vs_total);
   hipStream_t s = (hipStream_t)stream;
   if (wide) {
-    if (a.kd != nullptr) return verify::launch_wide<true, false, true, true>(a, s);
-    return a.window > 0 ? verify::launch_wide<true, false, true>(a, s) : verify::launch_wide<true>(a, s);
+    if (a.kd != nullptr) return verify::launch_wide<true, false, true, true>(a, head_dim, s);
+    return a.window > 0 ? verify::launch_wide<true, false, true>(a, head_dim, s) : verify::launch_wide<true>(a, head_dim, s);
   }
   if (a.window > 0)
     return head_dim == 128 ? verify::launch<128, true, true>(a, s) : verify::launch<256, true, true>(a, s);
@@ -2190,15 +2216,15 @@ extern "C" int s8kv_attn_varlen_f16(const void* q, const void* k, const void* v,
   // q loads (16 bytes) and output stores (8 bytes) are aligned
   // (and K and V tiles keep 32-bit offsets)
   auto tile_fits = [](int64_t stride_t) { return stride_t >= 0 && stride_t <= 1 << 25; };
-  const bool wide = head_dim == 128 && (uintptr_t)q % 16 == 0 && q_stride_t % 8 == 0 && q_stride_h % 8 == 0 &&
+  const bool wide = head_dim != 64 && (uintptr_t)q % 16 == 0 && q_stride_t % 8 == 0 && q_stride_h % 8 == 0 &&
                     (uintptr_t)out % 8 == 0 && o_stride_t % 4 == 0 && o_stride_h % 4 == 0 && tile_fits(k_stride_t) &&
                     tile_fits(v_stride_t);
   if (wide)
-    a.n_qblocks = (a.group * max_seqlen_q + verify::rows_per_wg(128, false, true, a.group * max_seqlen_q) - 1) /
-                  verify::rows_per_wg(128, false, true, a.group * max_seqlen_q);
+    a.n_qblocks = (a.group * max_seqlen_q + verify::rows_per_wg(head_dim, false, true, a.group * max_seqlen_q) - 1) /
+                  verify::rows_per_wg(head_dim, false, true, a.group * max_seqlen_q);
   if (window_left > 0) {  // query s sees keys (s + nk - nq - window_left, s + nk - nq]: window_left keys
     a.window = window_left - 1;  // the kernel's band: keys >= s + nk - nq - window
-    if (wide) return verify::launch_wide<false, true, true>(a, s);
+    if (wide) return verify::launch_wide<false, true, true>(a, head_dim, s);
     switch (head_dim) {
       case 64: return verify::launch<64, false, true, true>(a, s);
       case 128: return verify::launch<128, false, true, true>(a, s);
@@ -2206,7 +2232,7 @@ extern "C" int s8kv_attn_varlen_f16(const void* q, const void* k, const void* v,
     }
     return S8KV_ERR_UNSUPPORTED;
   }
-  if (wide) return verify::launch_wide<false, true>(a, s);
+  if (wide) return verify::launch_wide<false, true>(a, head_dim, s);
   switch (head_dim) {
     case 64: return verify::launch<64, false, false, true>(a, s);
     case 128: return verify::launch<128, false, false, true>(a, s);

@@ -88,14 +88,15 @@ def test_equal_splits_of_ragged_rows(kind, d, window):
 
 @pytest.mark.parametrize("kind", ["int8", "k8v3"])
 @pytest.mark.parametrize("bs,nq,tree", [(4, 40, False), (8, 64, True), (32, 64, True), (256, 33, False)])
+@pytest.mark.parametrize("d", [128, 256])
 @pytest.mark.parametrize("window", [None, 40])
-def test_more_than_128_rows(kind, bs, nq, tree, window):
-    """Rows enough for 8-wave workgroups (G 4): prefixes that start the drafts
+def test_more_than_128_rows(kind, bs, nq, tree, d, window):
+    """Rows enough for 8-wave workgroups (G 4, head_dim 128; at 256 two blocks of 4): prefixes that start the drafts
     at every kind of place in a 32-key tile, one to three tiles in all, odd and
     even tile counts, more blocks than are looked up at a time (bs 4, 2,047
     keys and up), blocks smaller than a tile, and waves without a live row."""
     prefix = [0, 1, 31, 32, 33, 64, 95, 2047 + 5 * bs, 700]
-    _check(300 + bs + nq, kind, 8, 2, 128, bs, prefix, nq, f"{kind} bs={bs} nq={nq} tree={tree} window={window}",
+    _check(300 + bs + nq, kind, 8, 2, d, bs, prefix, nq, f"{kind} D={d} bs={bs} nq={nq} tree={tree} window={window}",
            query_lens=[nq, nq, 1, nq - 1, nq, 9, nq, nq, 0], window=window, tree=tree)
 
 
