@@ -105,8 +105,8 @@ struct VerifyArgs {
   int max_context_len;
   int n_qblocks;              // query blocks (rows_per_wg rows each) per (sequence, KV head)
   // split of the key range: workgroup split sp of a (sequence, KV head, query
-  // block) attends keys split_keys * sp .. of the block's range (a short row
-  // has fewer non-empty splits) and writes unnormalized partials (acc[D],
+  // block) attends the sp-th of the block's equal pieces of at most split_keys
+  // keys (a short row has fewer) and writes unnormalized partials (acc[D],
   // m_ref, l per row, pitch D + 4 floats, part_rows rows per unit) of its live
   // 16- or 32-row groups to part; a second kernel combines them.  splits == 1:
   // the workgroup writes the output itself.
@@ -154,11 +154,18 @@ __device__ __forceinline__ Unit unit_of(const VerifyArgs& a, int id) {
   return {pg * g + (rem & (g - 1)), u - sp * a.n_qblocks, sp};
 }
 
-// Split sp of a block whose keys are [lo, end) (lo tile-aligned): [k_lo, k_hi).
+// Keys per split of a block that has `keys`: as few equal pieces (whole tiles)
+// as split_keys allows.
+__device__ __forceinline__ int split_piece(const VerifyArgs& a, int keys) {
+  const int n = max(1, (keys + a.split_keys - 1) / a.split_keys);
+  return ((keys + n - 1) / n + kTile - 1) & ~(kTile - 1);
+}
+// Split sp of a block whose keys are [k_lo, end) (k_lo tile-aligned): [k_lo, k_hi).
 __device__ __forceinline__ void split_range(const VerifyArgs& a, int sp, int end, int& k_lo, int& k_hi) {
   if (a.splits == 1) return;
-  k_lo += sp * a.split_keys;
-  if (sp + 1 < a.splits) k_hi = min(end, k_lo + a.split_keys);
+  const int piece = split_piece(a, max(0, end - k_lo));
+  k_lo += sp * piece;
+  k_hi = min(end, k_lo + piece);
 }
 
 // Position of tile key tt (0..31) in the LDS V tile: lane group g's eight
@@ -857,9 +864,10 @@ __device__ __forceinline__ void split_pair(float w0, float w1, uint32_t& hi, uin
   lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(l0, l1));
 }
 
-template <int D, bool K8V3, bool EIGHT>
+template <int D, bool K8V3, bool EIGHT, bool NARROW = false>
 struct WideCfg {
   static_assert(D == 128 || (D == 256 && !EIGHT), "head_dim 256: 4 waves");
+  static_assert(!EIGHT || !NARROW, "narrow workgroups have 4 waves");
   // EIGHT (calls with more than 128 query rows per sequence and KV head):
   // 8 waves (256 rows) per workgroup, one workgroup per CU, so twice the rows
   // share each tile's staging (K8V3: code expansion); else 4 waves, two per CU
@@ -868,7 +876,9 @@ struct WideCfg {
   // accumulators and q hi + lo (128 each)
   static constexpr int WG_PER_CU = D == 256 ? 1 : 8 / WAVES;
   static constexpr int THREADS = 64 * WAVES;
-  static constexpr int ROWS = 32 * WAVES;  // query rows per workgroup
+  // NARROW (calls with at most 32 query rows per sequence and KV head): every
+  // wave holds the same 32 rows and takes every fourth tile
+  static constexpr int ROWS = NARROW ? 32 : 32 * WAVES;  // query rows per workgroup
   static constexpr int KROW = 2 * D + 16;  // LDS pitch of an fp16 K row (8 consecutive rows: distinct 16-byte slots)
   static constexpr int VROW = 2 * D + 32;  // LDS pitch of an fp16 V row (4 rows of a transpose read: distinct banks)
   static constexpr int KBYTES = kTile * KROW;
@@ -877,13 +887,15 @@ struct WideCfg {
   static constexpr int SBYTES = (1 + NB) * kTile * 4;  // k_scale, then the V scales of each block
   static constexpr int BUF = KBYTES + VBYTES + SBYTES;
   static constexpr int PARTS = D / 16;   // 16-byte int8 chunks of a key's K (or V); K8V3: half code groups
-  static constexpr int NCH = EIGHT ? 1 : kTile * PARTS / THREADS;  // of a tile, per thread (EIGHT: K, or V)
+  static constexpr int NCH = EIGHT ? 1 : kTile * PARTS / (NARROW ? 64 : THREADS);  // of a tile, per thread (EIGHT: K, or V)
   static constexpr int NG = D / 32;      // K8V3: 32-value code groups per key
   static constexpr int WORDS = 3 * NG;   // K8V3: packed words per key
   static constexpr int HALF = D / 2;     // dims a lane holds of q and takes of a K row
   static constexpr int NM = D / 16;      // QK MFMAs (of hi or lo)
   static constexpr int NT = D / 32;      // 32-dim tiles of the output
-  static constexpr int SMEM = 2 * BUF + kMaxSubBlocks * 4;
+  static constexpr int BUFS = NARROW ? 4 : 2;  // tile buffers (NARROW: one per wave)
+  static constexpr int SMEM = BUFS * BUF + kMaxSubBlocks * 4;
+  static_assert(!NARROW || kTile * D * 4 + 2 * kTile * 4 <= BUF, "a wave's accumulators, maxima and sums fit its buffer");
   // window verify with fresh drafts: the low fp16 part of the drafts' K per buffer
   static constexpr int KLO_OFF = (SMEM + 15) / 16 * 16;
   static constexpr int SMEM_WIN = KLO_OFF + 2 * KBYTES;
@@ -896,16 +908,18 @@ struct WideCfg {
 // every row sees the last `window` prefix keys and the drafts, keys j >=
 // prefix - window, the drafts' K / V from the cache or (FRESH, a.kd set) from
 // the fresh fp32 K (rotated) and fp16 V rows of the drafts.
-template <int D, bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false, bool EIGHT = false>
+template <int D, bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false, bool EIGHT = false,
+          bool NARROW = false>
 __global__
 __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::WG_PER_CU)) void verify_wide_kernel(
     VerifyArgs a) {
+  static_assert(!NARROW || (!DENSE && !FRESH), "narrow: paged keys only");
   static_assert(!(DENSE && K8V3), "dense inputs: fp16 K / V");
   static_assert(!FRESH || (WIN && !DENSE), "fresh drafts: a paged window verify");
-  using C = WideCfg<D, K8V3, EIGHT>;
+  using C = WideCfg<D, K8V3, EIGHT, NARROW>;
   constexpr int NM = C::NM, NT = C::NT, NB = C::NB, PARTS = C::PARTS, HALF = C::HALF;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  int* bt_lds = reinterpret_cast<int*>(smem + 2 * C::BUF);
+  int* bt_lds = reinterpret_cast<int*>(smem + C::BUFS * C::BUF);
 
   const Unit unit = unit_of(a, blockIdx.x);
   const int qb = unit.qb, sp = unit.sp, p = unit.p;
@@ -915,6 +929,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row_wave = NARROW ? 0 : wave;  // the wave's 32 rows among the workgroup's
   const int j = lane & 31;  // this lane's query row within the wave (and the K row of its QK A operand)
   const int hf = lane >> 5;
 
@@ -949,7 +964,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
   split_range(a, sp, kv_end, k_lo, k_hi);
   if (a.splits > 1 && k_lo >= k_hi) return;  // no partial (the combine counts the splits with keys)
 
-  const int r = row0 + wave * 32 + j;
+  const int r = row0 + row_wave * 32 + j;
   const int pos = r / G;
   const int head = h * G + (r - pos * G);
   const bool row_live = pos < nq;
@@ -1286,10 +1301,134 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
   // the last block of a chunk) takes part in the tile loads, conversions and
   // barriers only; its rows are written as zeros.  The key loop is
   // instantiated for both kinds of wave, so neither carries the other's branch.
-  const bool wave_live = (row0 + wave * 32) / G < nq;
+  const bool wave_live = (row0 + row_wave * 32) / G < nq;
   auto key_loop = [&](auto live_tag) {
     constexpr bool LIVE = decltype(live_tag)::value;
-    if constexpr (EIGHT) {
+    if constexpr (NARROW) {
+      // Each wave stages and computes its own tiles (tile t of the range: wave
+      // t % 4) in its own buffer, without a barrier, one tile's loads ahead of
+      // the one in LDS: 8 waves a CU keep 67 KB in flight (head_dim 128).  With
+      // the four waves sharing each tile, three of them only staged for the
+      // one that had rows, and each tile cost its whole latency: 32 rows of 5
+      // queries (20 query rows a head), contexts of 256 .. 8,192, 130 -> 73 us.
+      const int sub = (int)min((int64_t)(kMaxSubBlocks - 2) << bs_log2, (int64_t)(k_hi - k_lo));
+      for (int u0 = k_lo; u0 < k_hi; u0 += sub) {
+        const int u1 = min(k_hi, u0 + sub);
+        const int fb = u0 >> bs_log2;
+        __syncthreads();  // previous users of bt_lds are done
+        for (int i = tid; i <= ((u1 - 1) >> bs_log2) - fb; i += C::THREADS) bt_lds[i] = bt_row[fb + i];
+        __syncthreads();
+        struct TileRegs {
+          u32x4_t k[C::NCH], v[C::NCH];
+          float s[NB];
+        } R;
+        auto load_tile = [&](int base) {
+          // one block holds the tile (bs >= 32): scalar offset of its first row
+          // (rows past the last key are read too, and masked; not their
+          // scales); else a row per lane
+          const int lim = u1 - 1 - base;  // the last key of the range, from the tile's first
+          const bool one = bs_log2 >= 5;
+          auto row_of = [&](int tt) -> uint32_t {
+            const int kk = base + min(tt, lim);
+            return (((uint32_t)bt_lds[(kk >> bs_log2) - fb] * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)kk & bsm);
+          };
+          const uint32_t row = one ? (uint32_t)__builtin_amdgcn_readfirstlane((int)row_of(0)) : 0u;
+          uint32_t at[C::NCH];
+          const int tk = lane & (kTile - 1);
+          uint32_t scale_at = (uint32_t)min(tk, lim);
+#pragma unroll
+          for (int i = 0; i < C::NCH; ++i) at[i] = (uint32_t)((lane + 64 * i) / PARTS);
+          if (!one) {
+            scale_at = row_of(tk);
+#pragma unroll
+            for (int i = 0; i < C::NCH; ++i) at[i] = row_of((lane + 64 * i) / PARTS);
+          }
+#pragma unroll
+          for (int i = 0; i < C::NCH; ++i) {
+            const uint32_t part = (uint32_t)((lane + 64 * i) % PARTS);
+            R.k[i] = bload128<kNT>(kc, at[i] * (uint32_t)D + part * 16u, row * (uint32_t)D);
+            if constexpr (K8V3) {
+              const u32x3_t w = bload96<kNT>(vc, at[i] * (uint32_t)(C::WORDS * 4) + (part >> 1) * 12u,
+                                             row * (uint32_t)(C::WORDS * 4));
+              R.v[i].x = w.x;
+              R.v[i].y = w.y;
+              R.v[i].z = w.z;
+            } else {
+              R.v[i] = bload128<kNT>(vc, at[i] * (uint32_t)D + part * 16u, row * (uint32_t)D);
+            }
+          }
+          // (NB 1: K scales in lanes 0..31, V's in 32..63; NB 2: K's, then V's two per lane)
+          if (lane < kTile) R.s[0] = __builtin_bit_cast(float, bload32(ks, scale_at * 4u, row * 4u));
+          else if (NB == 1) R.s[0] = __builtin_bit_cast(float, bload32(vs, scale_at * 4u, row * 4u));
+          if constexpr (NB == 2)
+            R.s[1] = __builtin_bit_cast(float, bload32(vs, (scale_at * NB + (uint32_t)(lane >> 5)) * 4u, row * (NB * 4u)));
+        };
+        auto store_tile = [&](int base) {
+#pragma unroll
+          for (int i = 0; i < C::NCH; ++i) {
+            const int ch = lane + 64 * i, tt = ch / PARTS;
+            store_k(wave, base, tt, ch % PARTS, R.k[i]);
+            store_v(wave, base, tt, ch, R.v[i]);
+          }
+          const int tk = lane & (kTile - 1);
+          if (NB == 1) store_scale(wave, base, tk, lane >> 5, R.s[0]);
+          else if (lane < kTile) store_scale(wave, base, tk, 0, R.s[0]);
+          if constexpr (NB == 2) store_scale(wave, base, tk, 1 + (lane >> 5), R.s[1]);
+        };
+        if constexpr (LIVE) {
+          int base = u0 + wave * kTile;
+          if (base < u1) load_tile(base);
+          for (; base < u1; base += 4 * kTile) {
+            store_tile(base);
+            // (the wave's LDS instructions run in order; the fences keep the compiler's order)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (base + 4 * kTile < u1) load_tile(base + 4 * kTile);
+            qk(wave);
+            weights(wave, base, hides(base));
+            pv(wave);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          }
+        }
+      }
+      // the four waves' sums: each wave's accumulators, maxima and sums to its
+      // buffer, then each wave adds a quarter of the dims of all rows
+      if constexpr (LIVE) {
+        l_run = sum_x32(l_run);
+        float* own = reinterpret_cast<float*>(smem + wave * C::BUF);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4_t*>(own + ((n * 4 + q) * 64 + lane) * 4) =
+                float4_t{acc[n][4 * q], acc[n][4 * q + 1], acc[n][4 * q + 2], acc[n][4 * q + 3]};
+        }
+        if (hf == 0) {
+          own[kTile * D + j] = m_ref;
+          own[kTile * D + kTile + j] = l_run;
+        }
+        __syncthreads();
+        float f[4], m[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) m[w] = reinterpret_cast<const float*>(smem + w * C::BUF)[kTile * D + j];
+        m_ref = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
+        l_run = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          f[w] = __builtin_amdgcn_exp2f(m[w] - m_ref);
+          l_run += f[w] * reinterpret_cast<const float*>(smem + w * C::BUF)[kTile * D + kTile + j];
+        }
+#pragma unroll
+        for (int c = 0; c < NT; ++c) {  // (into the first accumulators' registers: chunk wave * NT + c)
+          float4_t x = float4_t{};
+#pragma unroll
+          for (int w = 0; w < 4; ++w)
+            x += f[w] * *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(smem + w * C::BUF) +
+                                                           ((wave * NT + c) * 64 + lane) * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[c >> 2][4 * (c & 3) + e] = x[e];
+        }
+      }
+    } else if constexpr (EIGHT) {
       // The waves of a SIMD (wave w and w + 4) run half a tile apart: while
       // waves 0..3 issue a tile's MFMAs (PV of tile t - 1, QK of tile t), waves
       // 4..7 do the softmax of tile t - 1 and stage, then the other way
@@ -1568,20 +1707,24 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       key_loop(std::false_type{});
   }
 
-  const float l_tot = sum_x32(l_run);
+  const float l_tot = NARROW ? l_run : sum_x32(l_run);
+  // this lane's dims of row j: acc[n][4 q ..] are 32 n + 8 q + 4 hf .. + 3
+  // (NARROW: chunks 4 n + q of the wave's quarter)
+  constexpr int NOUT = NARROW ? NT / 4 : NT;
+  const int n0 = NARROW ? wave * NOUT : 0;
   // ---- split: this wave's unnormalized rows to the partials ----
   if (a.splits > 1) {
     if (!wave_live) return;  // (no row of the wave is read back)
-    const int rl = wave * 32 + j;
+    const int rl = row_wave * 32 + j;
     float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * a.part_rows + rl) * (D + 4);
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
+    for (int n = 0; n < NOUT; ++n) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4_t*>(pr + 32 * n + 8 * q + 4 * hf) =
+        *reinterpret_cast<float4_t*>(pr + 32 * (n0 + n) + 8 * q + 4 * hf) =
             float4_t{acc[n][4 * q], acc[n][4 * q + 1], acc[n][4 * q + 2], acc[n][4 * q + 3]};
     }
-    if (hf == 0) {
+    if (hf == 0 && n0 == 0) {
       pr[D] = m_ref;
       pr[D + 1] = l_tot;
     }
@@ -1594,13 +1737,13 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
     _Float16* op = DENSE ? a.out + (int64_t)(q0 + pos) * a.o_stride_t + (int64_t)head * a.o_stride_h
                          : a.out + (((int64_t)b * a.num_q_heads + head) * a.max_queries + pos) * D;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
+    for (int n = 0; n < NOUT; ++n) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         half4_t o;
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) o[rr] = (_Float16)(acc[n][4 * q + rr] * inv);
-        *reinterpret_cast<half4_t*>(op + 32 * n + 8 * q + 4 * hf) = o;
+        *reinterpret_cast<half4_t*>(op + 32 * (n0 + n) + 8 * q + 4 * hf) = o;
       }
     }
   }
@@ -1619,8 +1762,14 @@ static bool use_wide(int head_dim, bool big) { return (head_dim == 128 || head_d
 // rows: query rows per (sequence, KV head) -- group x max_queries; the wide
 // kernel takes 8-wave workgroups at head_dim 128 when they exceed one 4-wave block
 static bool wide_eight(int head_dim, int rows) { return head_dim == 128 && rows > WideCfg<128, false, false>::ROWS; }
+// ... and narrow ones when they fit one wave (one block either way, so only the
+// launch cares that dense calls and fresh drafts keep the 4-wave ones)
+static bool wide_narrow(int rows) { return rows <= WideCfg<128, false, false, true>::ROWS; }
 static int rows_per_wg(int head_dim, bool k8v3, bool wide, int rows) {
-  if (wide) return wide_eight(head_dim, rows) ? WideCfg<128, false, true>::ROWS : WideCfg<128, false, false>::ROWS;
+  if (wide)
+    return wide_eight(head_dim, rows) ? WideCfg<128, false, true>::ROWS
+           : wide_narrow(rows)        ? WideCfg<128, false, false, true>::ROWS
+                                      : WideCfg<128, false, false>::ROWS;
   return 16 * (k8v3 ? 8 : 4) * (head_dim <= 64 ? 2 : 1);
 }
 static int wg_per_cu(int head_dim, bool k8v3, bool wide, int rows) {
@@ -1663,7 +1812,8 @@ __global__ __launch_bounds__(kCombineThreads) void verify_combine_kernel(VerifyA
   const int prefix = max(0, a.prefix_lens[b]);
   const int end = min(prefix + (a.tree_mask ? nq : min(nq, (qb * ROWS + ROWS + G - 1) / G)), a.max_context_len);
   const int k_lo = a.window > 0 ? max(0, prefix - a.window) & ~(kTile - 1) : 0;
-  const int S = min(a.splits, (max(0, end - k_lo) + a.split_keys - 1) / a.split_keys);
+  const int keys = max(0, end - k_lo), piece = max(kTile, split_piece(a, keys));
+  const int S = (keys + piece - 1) / piece;
   const int64_t stride = (int64_t)a.part_rows * (D + 4);  // between splits of one row
   const float* row = a.part + ((int64_t)pq * a.splits * a.part_rows + rl) * (D + 4);
   // one pass: the running max rises batch by batch and rescales what is
@@ -1763,13 +1913,13 @@ static int launch(VerifyArgs& a, hipStream_t stream) {
                  : launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
 }
 
-template <int D, bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT>
+template <int D, bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT, bool NARROW>
 static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
-  using C = WideCfg<D, K8V3, EIGHT>;
+  using C = WideCfg<D, K8V3, EIGHT, NARROW>;
   constexpr int smem = FRESH ? C::SMEM_WIN : C::SMEM;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT, NARROW>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
       set_error("s8kv_verify: cannot set the dynamic LDS size");
       return S8KV_ERR_LAUNCH;
@@ -1782,7 +1932,7 @@ static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
     set_error("s8kv_verify: grid too large");
     return S8KV_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT>), dim3((unsigned)grid), dim3(C::THREADS), smem,
+  hipLaunchKernelGGL((verify_wide_kernel<D, K8V3, DENSE, WIN, FRESH, EIGHT, NARROW>), dim3((unsigned)grid), dim3(C::THREADS), smem,
                      stream, a);
   if (a.splits > 1) {
     const int rc = check_launch("s8kv_verify");
@@ -1798,9 +1948,15 @@ static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
 // rule (rows_per_wg, wg_per_cu)
 template <bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false>
 static int launch_wide(VerifyArgs& a, int head_dim, hipStream_t stream) {
-  if (head_dim == 256) return launch_wide_impl<256, K8V3, DENSE, WIN, FRESH, false>(a, stream);
-  if (wide_eight(head_dim, a.group * a.max_queries)) return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, true>(a, stream);
-  return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, false>(a, stream);
+  const int rows = a.group * a.max_queries;
+  if constexpr (!DENSE && !FRESH) {
+    if (wide_narrow(rows))
+      return head_dim == 256 ? launch_wide_impl<256, K8V3, DENSE, WIN, FRESH, false, true>(a, stream)
+                             : launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, false, true>(a, stream);
+  }
+  if (head_dim == 256) return launch_wide_impl<256, K8V3, DENSE, WIN, FRESH, false, false>(a, stream);
+  if (wide_eight(head_dim, rows)) return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, true, false>(a, stream);
+  return launch_wide_impl<128, K8V3, DENSE, WIN, FRESH, false, false>(a, stream);
 }
 
 }  // namespace verify
@@ -1817,9 +1973,9 @@ struct FreshDrafts {
   int64_t v_stride[3];
 };
 
-// Key-range split of the paged verify: the units of a (sequence, KV head,
-// query block) take an equal number of keys, so a short row has fewer of them
-// and the longest row's share bounds the launch.  Two reasons to split:
+// Key-range split of the paged verify: a (sequence, KV head, query block) is
+// cut into the fewest equal pieces within a length that all rows share, so a
+// short row has fewer and the longest row's share bounds the launch.  Two reasons to split:
 //  * a launch with fewer workgroups than the GPU keeps resident leaves CUs
 //    idle for the whole call -- batch-1 speculative decoding with a long context
 //    is the common case -- so units are split until about that many exist,
@@ -1830,9 +1986,14 @@ struct FreshDrafts {
 //    longest one runs alone at the end.  Splits of at least kMinSplitKeys keys,
 //    and 32 keys per query row (a split writes and the combine reads 1 KB a
 //    row, against the 270 bytes a key and head that it streams), up to
-//    kBalanceRounds units per resident workgroup, keep every CU busy.  Batch
-//    32, 5 queries, 8 KV heads, contexts of 256 .. 8,192 (mean 2,300): 2
-//    halves of each row 184.7 us a call, equal splits of 640 keys 132.9.
+//    kBalanceRounds units per resident workgroup and whole rounds of them.
+// Narrow workgroups (at most 32 query rows) read 128 keys at a time, so they
+// are cut finer: to one per CU down to 128 keys each, to two per CU down to
+// 512, and to six per CU -- two rounds of them when the mean row is a third of
+// the longest -- down to 1,024.  us a call: 32 rows of 256 .. 8,192 (mean
+// 2,300), 8 heads, in 2 / 3 / 6 / 12 splits: 91 / 71 / 73 / 83; one row of 4,647,
+// 4 heads, in 4 / 12 / 36: 27 / 24 / 24; 17 rows of up to 3,018, 2 heads, in 3 /
+// 6 / 16: 39 / 32 / 40.
 // One workgroup never accumulates more than kMaxSplitKeys keys, which bounds
 // the rounding of its fp32 sums.  s8kv_verify_set_splits overrides the count
 // (diagnostics).
@@ -1845,12 +2006,18 @@ static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int ke
                               int rows, int rows_wg) {
   const int64_t natural = (int64_t)batch * num_kv_heads * n_qblocks;
   const int64_t resident = (int64_t)verify::wg_per_cu(head_dim, k8v3, wide, rows) * device_cus();
+  auto units = [&](int64_t total, int64_t least_keys) {  // splits that make `total` units, each of least_keys or more
+    return std::min<int64_t>((total + natural - 1) / natural, keys / least_keys);
+  };
   int64_t s = natural < resident ? (resident + natural - 1) / natural : 1;
+  const int64_t fill = s;
   s = std::min<int64_t>(s, std::max(1, keys / kMinSplitKeys));
   if (batch > 1) {
     const int64_t least = std::max(kMinSplitKeys, 32 * std::min(rows, rows_wg));
-    s = std::max(s, std::min(keys / least, (kBalanceRounds * resident + natural - 1) / natural));
+    s = std::max(s, units(kBalanceRounds * resident, least) / fill * fill);
   }
+  if (wide && verify::wide_narrow(rows))
+    s = std::max({units(device_cus(), 128), units(2 * device_cus(), 512), units(6 * device_cus(), 1024)});
   s = std::max<int64_t>(s, ((int64_t)keys + kMaxSplitKeys - 1) / kMaxSplitKeys);
   const int forced = g_verify_splits.load();
   if (forced > 0) s = forced;

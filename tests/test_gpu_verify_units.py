@@ -77,13 +77,30 @@ def test_dense_units_of_any_pair_count(batch, hkv):
 
 @pytest.mark.parametrize("kind,d", [("int8", 128), ("int8", 64), ("int8", 256), ("k8v3", 128), ("k8v3", 256)])
 @pytest.mark.parametrize("window", [None, 700])
-def test_equal_splits_of_ragged_rows(kind, d, window):
+@pytest.mark.parametrize("bs", [4, 32])
+@pytest.mark.parametrize("splits", [0, 1])
+def test_equal_splits_of_ragged_rows(kind, d, window, bs, splits):
     """The planned split of a batch of short and long rows with few queries:
     rows ending at, one below and one past a split's last key and tile, an
-    empty prefix, and rows whose queries are fewer than the call's."""
+    empty prefix, and rows whose queries are fewer than the call's; and the
+    same unsplit (at 4-token blocks more blocks than are looked up at a time)."""
     prefix, nq = [2600, 0, 511, 512, 513, 1023, 1024, 31, 33], 5
     lens = [5, 5, 1, 5, 0, 2, 5, 5, 3]
-    _check(80 + d, kind, 8, 2, d, 32, prefix, nq, f"{kind} D={d} window={window}", query_lens=lens, window=window)
+    lib = _lib.load()
+    _lib.check(lib.s8kv_verify_set_splits(splits), "set_splits")
+    try:
+        _check(80 + d, kind, 8, 2, d, bs, prefix, nq, f"{kind} D={d} window={window}", query_lens=lens, window=window)
+    finally:
+        lib.s8kv_verify_set_splits(0)
+
+
+@pytest.mark.parametrize("kind,d", [("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
+@pytest.mark.parametrize("hq,nq", [(8, 8), (8, 9), (2, 32), (2, 33), (4, 1)])
+def test_rows_around_one_wave(kind, d, hq, nq):
+    """32 query rows a KV head (the narrow workgroups' most), one group more,
+    and one query; trees and contexts from empty to a few tiles per wave."""
+    _check(700 + d + nq, kind, hq, 2, d, 16, [0, 5, 128, 129, 300], nq, f"{kind} D={d} {hq}/2 heads x {nq}",
+           query_lens=[nq, 1, nq, 0, nq], tree=True)
 
 
 @pytest.mark.parametrize("kind", ["int8", "k8v3"])
