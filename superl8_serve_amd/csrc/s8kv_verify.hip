@@ -826,7 +826,7 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
 }
 
 // ---------------------------------------------------------------------------
-// Wide verify (head_dim 128 and 256; paged int8 or K8V3 cache, or dense): 32 query rows per wave
+// Wide verify (paged int8 or K8V3 cache, or dense): 32 query rows per wave
 // on v_mfma_f32_32x32x16_f16, so every K and V operand a wave reads from LDS
 // feeds twice the MFMAs of a 16-row wave.  Lane (j = lane % 32, hf = lane /
 // 32) holds query row j of its wave (head_dim D):
@@ -866,7 +866,7 @@ __device__ __forceinline__ void split_pair(float w0, float w1, uint32_t& hi, uin
 
 template <int D, bool K8V3, bool EIGHT, bool NARROW = false>
 struct WideCfg {
-  static_assert(D == 128 || (D == 256 && !EIGHT), "head_dim 256: 4 waves");
+  static_assert(D == 128 || ((D == 64 || D == 256) && !EIGHT), "8 waves at head_dim 128 only");
   static_assert(!EIGHT || !NARROW, "narrow workgroups have 4 waves");
   // EIGHT (calls with more than 128 query rows per sequence and KV head):
   // 8 waves (256 rows) per workgroup, one workgroup per CU, so twice the rows
@@ -874,7 +874,7 @@ struct WideCfg {
   static constexpr int WAVES = EIGHT ? 8 : 4;
   // head_dim 256: one wave per SIMD, whose 512 registers hold the row group's
   // accumulators and q hi + lo (128 each)
-  static constexpr int WG_PER_CU = D == 256 ? 1 : 8 / WAVES;
+  static constexpr int WG_PER_CU = D == 256 ? 1 : D == 64 ? 3 : 8 / WAVES;
   static constexpr int THREADS = 64 * WAVES;
   // NARROW (calls with at most 32 query rows per sequence and KV head): every
   // wave holds the same 32 rows and takes every fourth tile
@@ -887,7 +887,9 @@ struct WideCfg {
   static constexpr int SBYTES = (1 + NB) * kTile * 4;  // k_scale, then the V scales of each block
   static constexpr int BUF = KBYTES + VBYTES + SBYTES;
   static constexpr int PARTS = D / 16;   // 16-byte int8 chunks of a key's K (or V); K8V3: half code groups
-  static constexpr int NCH = EIGHT ? 1 : kTile * PARTS / (NARROW ? 64 : THREADS);  // of a tile, per thread (EIGHT: K, or V)
+  static constexpr int CHUNKS = kTile * PARTS;
+  // of a tile, per thread (EIGHT: K, or V; 4 waves at head_dim 64: of the first half of the threads)
+  static constexpr int NCH = EIGHT ? 1 : NARROW ? CHUNKS / 64 : (CHUNKS + THREADS - 1) / THREADS;
   static constexpr int NG = D / 32;      // K8V3: 32-value code groups per key
   static constexpr int WORDS = 3 * NG;   // K8V3: packed words per key
   static constexpr int HALF = D / 2;     // dims a lane holds of q and takes of a K row
@@ -1140,11 +1142,12 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
     sc = float16_t{};
 #pragma unroll
     for (int m0 = 0; m0 < NM; m0 += 8) {
-      half8_t ka[8];
+      constexpr int MB = NM < 8 ? NM : 8;
+      half8_t ka[MB];
 #pragma unroll
-      for (int m = 0; m < 8; ++m) ka[m] = read_ka(buf, m0 + m);
+      for (int m = 0; m < MB; ++m) ka[m] = read_ka(buf, m0 + m);
 #pragma unroll
-      for (int m = 0; m < 8; ++m) {
+      for (int m = 0; m < MB; ++m) {
         sc = mfma32x32x16(ka[m], qhi[m0 + m], sc);
         if constexpr (!DENSE) sc = mfma32x32x16(ka[m], qlo[m0 + m], sc);
       }
@@ -1613,7 +1616,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       };
       // 16-byte chunks of the tile's K and V per thread: int8 (K8V3 V: a half
       // code group's three words), or fp16
-      constexpr int NCH = DENSE ? 2 * C::NCH : C::NCH;
+      constexpr int NCH = DENSE ? 2 * C::CHUNKS / C::THREADS : C::NCH;
       struct TileRegs {
         u32x4_t k[NCH], v[NCH];
         float s;
@@ -1634,6 +1637,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
           const int ch = tid + i * C::THREADS, tt = ch / PARTS, part = ch % PARTS;
+          if (C::CHUNKS < C::THREADS && ch >= C::CHUNKS) continue;
           const uint32_t row = row_of(base + tt);
           R.k[i] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
           if constexpr (K8V3) {
@@ -1661,7 +1665,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
             const int tt = ch / (2 * PARTS), part = ch % (2 * PARTS);
             *reinterpret_cast<u32x4_t*>(kb + tt * C::KROW + part * 16) = R.k[i];
             *reinterpret_cast<u32x4_t*>(kb + C::KBYTES + tt * C::VROW + part * 16) = R.v[i];
-          } else {
+          } else if (C::CHUNKS >= C::THREADS || ch < C::CHUNKS) {
             const int tt = ch / PARTS;
             store_k(buf, base, tt, ch % PARTS, R.k[i]);
             store_v(buf, base, tt, ch, R.v[i]);
@@ -1708,23 +1712,23 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
   }
 
   const float l_tot = NARROW ? l_run : sum_x32(l_run);
-  // this lane's dims of row j: acc[n][4 q ..] are 32 n + 8 q + 4 hf .. + 3
-  // (NARROW: chunks 4 n + q of the wave's quarter)
-  constexpr int NOUT = NARROW ? NT / 4 : NT;
-  const int n0 = NARROW ? wave * NOUT : 0;
+  // this lane's dims of row j, in chunks: acc[c / 4][4 (c % 4) ..] are dims 8 c
+  // + 4 hf .. + 3
+  // (NARROW: 4 * NT chunks over 4 waves: NT each, from chunk wave * NT on)
+  constexpr int NCHUNK = NARROW ? NT : 4 * NT;
+  const int c0 = NARROW ? wave * NT : 0;
   // ---- split: this wave's unnormalized rows to the partials ----
   if (a.splits > 1) {
     if (!wave_live) return;  // (no row of the wave is read back)
     const int rl = row_wave * 32 + j;
     float* pr = a.part + ((((int64_t)p * a.n_qblocks + qb) * a.splits + sp) * a.part_rows + rl) * (D + 4);
 #pragma unroll
-    for (int n = 0; n < NOUT; ++n) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4_t*>(pr + 32 * (n0 + n) + 8 * q + 4 * hf) =
-            float4_t{acc[n][4 * q], acc[n][4 * q + 1], acc[n][4 * q + 2], acc[n][4 * q + 3]};
+    for (int c = 0; c < NCHUNK; ++c) {
+      const int n = c >> 2, q = c & 3;
+      *reinterpret_cast<float4_t*>(pr + 8 * (c0 + c) + 4 * hf) =
+          float4_t{acc[n][4 * q], acc[n][4 * q + 1], acc[n][4 * q + 2], acc[n][4 * q + 3]};
     }
-    if (hf == 0 && n0 == 0) {
+    if (hf == 0 && c0 == 0) {
       pr[D] = m_ref;
       pr[D + 1] = l_tot;
     }
@@ -1737,19 +1741,16 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
     _Float16* op = DENSE ? a.out + (int64_t)(q0 + pos) * a.o_stride_t + (int64_t)head * a.o_stride_h
                          : a.out + (((int64_t)b * a.num_q_heads + head) * a.max_queries + pos) * D;
 #pragma unroll
-    for (int n = 0; n < NOUT; ++n) {
+    for (int c = 0; c < NCHUNK; ++c) {
+      half4_t o;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        half4_t o;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) o[rr] = (_Float16)(acc[n][4 * q + rr] * inv);
-        *reinterpret_cast<half4_t*>(op + 32 * (n0 + n) + 8 * q + 4 * hf) = o;
-      }
+      for (int rr = 0; rr < 4; ++rr) o[rr] = (_Float16)(acc[c >> 2][4 * (c & 3) + rr] * inv);
+      *reinterpret_cast<half4_t*>(op + 8 * (c0 + c) + 4 * hf) = o;
     }
   }
 }
 
-// The wide kernel serves the paged head_dim-128 and -256 calls whose tensors
+// The wide kernel serves the paged calls whose tensors
 // fit 32-bit offsets (no per-tile descriptor rebasing), with or without a
 // window.  Head_dim 256 in the 16-row kernel: its accumulators and q hi + lo
 // left no registers at two waves per SIMD (over 400 bytes of spills a lane);
@@ -1758,7 +1759,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
 // Query rows per workgroup at this head_dim and layout (Cfg<D, K8V3>::ROWS,
 // or WideCfg::ROWS for the wide kernel), and the workgroups a CU keeps
 // resident (the kernels' launch bounds).
-static bool use_wide(int head_dim, bool big) { return (head_dim == 128 || head_dim == 256) && !big; }
+static bool use_wide(bool big) { return !big; }
 // rows: query rows per (sequence, KV head) -- group x max_queries; the wide
 // kernel takes 8-wave workgroups at head_dim 128 when they exceed one 4-wave block
 static bool wide_eight(int head_dim, int rows) { return head_dim == 128 && rows > WideCfg<128, false, false>::ROWS; }
@@ -1773,7 +1774,8 @@ static int rows_per_wg(int head_dim, bool k8v3, bool wide, int rows) {
   return 16 * (k8v3 ? 8 : 4) * (head_dim <= 64 ? 2 : 1);
 }
 static int wg_per_cu(int head_dim, bool k8v3, bool wide, int rows) {
-  return wide ? (wide_eight(head_dim, rows) || head_dim == 256 ? 1 : 2) : (k8v3 ? 1 : 2);
+  if (wide) return wide_eight(head_dim, rows) || head_dim == 256 ? 1 : head_dim == 64 ? 3 : 2;
+  return k8v3 ? 1 : 2;
 }
 
 // Combine of a split verify: one thread per (row, 4 dims) of a (sequence,
@@ -1906,11 +1908,8 @@ template <int D, bool K8V3, bool WIN = false, bool DENSE = false>
 static int launch(VerifyArgs& a, hipStream_t stream) {
   if constexpr (DENSE)
     return launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
-  else if constexpr (D >= 128)  // (the wide kernel serves the others)
+  else  // (the wide kernel serves the others)
     return launch_impl<D, K8V3, WIN, DENSE, true>(a, stream);
-  else
-    return a.big ? launch_impl<D, K8V3, WIN, DENSE, true>(a, stream)
-                 : launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
 }
 
 template <int D, bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT, bool NARROW>
@@ -1949,6 +1948,13 @@ static int launch_wide_impl(VerifyArgs& a, hipStream_t stream) {
 template <bool K8V3, bool DENSE = false, bool WIN = false, bool FRESH = false>
 static int launch_wide(VerifyArgs& a, int head_dim, hipStream_t stream) {
   const int rows = a.group * a.max_queries;
+  if constexpr (!K8V3) {
+    if (head_dim == 64) {
+      if constexpr (!DENSE && !FRESH)
+        if (wide_narrow(rows)) return launch_wide_impl<64, K8V3, DENSE, WIN, FRESH, false, true>(a, stream);
+      return launch_wide_impl<64, K8V3, DENSE, WIN, FRESH, false, false>(a, stream);
+    }
+  }
   if constexpr (!DENSE && !FRESH) {
     if (wide_narrow(rows))
       return head_dim == 256 ? launch_wide_impl<256, K8V3, DENSE, WIN, FRESH, false, true>(a, stream)
@@ -2040,7 +2046,6 @@ extern "C" int64_t s8kv_verify_workspace_size(int batch, int num_q_heads, int nu
   int64_t need = 0;
   for (const bool k8v3 : {false, true}) {
     for (const bool wide : {false, true}) {
-      if (wide && head_dim == 64) continue;
       const int rows = num_q_heads / num_kv_heads * max_queries;
       const int rows_wg = verify::rows_per_wg(head_dim, k8v3, wide, rows);
       const int n_qblocks = (rows + rows_wg - 1) / rows_wg;
@@ -2137,7 +2142,7 @@ static int verify_setup(verify::VerifyArgs& a, const void* q, int batch, int num
   a.tree_mask = tree_mask;
   a.bs_log2 = log2i(block_size);
   a.max_context_len = max_context_len;
-  const int rows_wg = verify::rows_per_wg(head_dim, k8v3, verify::use_wide(head_dim, a.big), a.group * max_queries);
+  const int rows_wg = verify::rows_per_wg(head_dim, k8v3, verify::use_wide(a.big), a.group * max_queries);
   a.n_qblocks = (a.group * max_queries + rows_wg - 1) / rows_wg;
   a.qscale = (float)((double)scale * 1.4426950408889634 / __builtin_sqrt((double)head_dim));
   a.out = (_Float16*)out;
@@ -2162,7 +2167,7 @@ static int verify_int8_impl(const void* q, int batch, int num_q_heads, int num_k
                               prefix_lens, query_lens, tree_mask, max_context_len, scale, out, false);
   if (rc != S8KV_OK) return rc;
   a.window = window;
-  const bool wide = verify::use_wide(head_dim, a.big);
+  const bool wide = verify::use_wide(a.big);
   if (const int rc = verify_use_workspace(a, head_dim, false, wide, workspace, workspace_bytes)) return rc;
   if (fresh_k) {
     S8KV_REQUIRE(fresh->v != nullptr && window > 0, S8KV_ERR_INVALID, "verify: fresh drafts need V and a window");
@@ -2260,7 +2265,7 @@ static int verify_k8v3_impl(const void* q, int batch, int num_q_heads, int num_k
                               prefix_lens, query_lens, tree_mask, max_context_len, scale, out, true);
   if (rc != S8KV_OK) return rc;
   a.window = window;
-  const bool wide = verify::use_wide(head_dim, a.big);
+  const bool wide = verify::use_wide(a.big);
   if (const int rc = verify_use_workspace(a, head_dim, true, wide, workspace, workspace_bytes)) return rc;
   if (fresh_k) {
     S8KV_REQUIRE(fresh->v != nullptr && window > 0, S8KV_ERR_INVALID, "verify: fresh drafts need V and a window");
@@ -2379,11 +2384,11 @@ extern "C" int s8kv_attn_varlen_f16(const void* q, const void* k, const void* v,
   a.causal = causal ? 1 : 0;
   a.out = (_Float16*)out;
   hipStream_t s = (hipStream_t)stream;
-  // head_dim 128: the wide kernel (32 query rows per wave) when its vector
+  // the wide kernel (32 query rows per wave) when its vector
   // q loads (16 bytes) and output stores (8 bytes) are aligned
   // (and K and V tiles keep 32-bit offsets)
   auto tile_fits = [](int64_t stride_t) { return stride_t >= 0 && stride_t <= 1 << 25; };
-  const bool wide = head_dim != 64 && (uintptr_t)q % 16 == 0 && q_stride_t % 8 == 0 && q_stride_h % 8 == 0 &&
+  const bool wide = (uintptr_t)q % 16 == 0 && q_stride_t % 8 == 0 && q_stride_h % 8 == 0 &&
                     (uintptr_t)out % 8 == 0 && o_stride_t % 4 == 0 && o_stride_h % 4 == 0 && tile_fits(k_stride_t) &&
                     tile_fits(v_stride_t);
   if (wide)

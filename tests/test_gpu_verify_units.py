@@ -58,12 +58,13 @@ def test_every_unit_of_any_pair_count(batch, hkv, d):
            f"{batch} x {hkv} pairs, D={d}")
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("batch,hkv", [(1, 2), (7, 1)])
-def test_dense_units_of_any_pair_count(batch, hkv):
+def test_dense_units_of_any_pair_count(batch, hkv, d):
     rng = np.random.default_rng(60 + batch)
     lens = [400 - 53 * b for b in range(batch)]
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
-    hq, d = 4 * hkv, 128
+    hq = 4 * hkv
     q, k, v = (rng.standard_normal((cu[-1], h, d)).astype(np.float16) for h in (hq, hkv, hkv))
     out = to_np(ops.attn_varlen(t(q), t(k), t(v), t(cu), t(cu), max(lens), max(lens), causal=True,
                                 scale=d ** -0.5).float())
@@ -94,7 +95,7 @@ def test_equal_splits_of_ragged_rows(kind, d, window, bs, splits):
         lib.s8kv_verify_set_splits(0)
 
 
-@pytest.mark.parametrize("kind,d", [("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
+@pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
 @pytest.mark.parametrize("hq,nq", [(8, 8), (8, 9), (2, 32), (2, 33), (4, 1)])
 def test_rows_around_one_wave(kind, d, hq, nq):
     """32 query rows a KV head (the narrow workgroups' most), one group more,
@@ -103,12 +104,11 @@ def test_rows_around_one_wave(kind, d, hq, nq):
            query_lens=[nq, 1, nq, 0, nq], tree=True)
 
 
-@pytest.mark.parametrize("kind", ["int8", "k8v3"])
+@pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
 @pytest.mark.parametrize("bs,nq,tree", [(4, 40, False), (8, 64, True), (32, 64, True), (256, 33, False)])
-@pytest.mark.parametrize("d", [128, 256])
 @pytest.mark.parametrize("window", [None, 40])
-def test_more_than_128_rows(kind, bs, nq, tree, d, window):
-    """Rows enough for 8-wave workgroups (G 4, head_dim 128; at 256 two blocks of 4): prefixes that start the drafts
+def test_more_than_128_rows(kind, d, bs, nq, tree, window):
+    """Rows enough for 8-wave workgroups (G 4, head_dim 128; else two blocks of 4): prefixes that start the drafts
     at every kind of place in a 32-key tile, one to three tiles in all, odd and
     even tile counts, more blocks than are looked up at a time (bs 4, 2,047
     keys and up), blocks smaller than a tile, and waves without a live row."""
