@@ -59,7 +59,7 @@ def test_every_unit_of_any_pair_count(batch, hkv, d):
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
-@pytest.mark.parametrize("batch,hkv", [(1, 2), (7, 1)])
+@pytest.mark.parametrize("batch,hkv", [(1, 2), (7, 1), (8, 16)])  # (8, 16): enough pairs for 256-row blocks
 def test_dense_units_of_any_pair_count(batch, hkv, d):
     rng = np.random.default_rng(60 + batch)
     lens = [400 - 53 * b for b in range(batch)]
