@@ -46,12 +46,16 @@ __all__ = [
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # (the raw handle of torch.cuda.current_stream(t.device), without its Stream object: 2.1 -> 0.2 us)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
-def _require(cond: bool, msg: str, exc=ValueError) -> None:
+def _require(cond: bool, msg, exc=ValueError) -> None:
+    """Raise ``exc`` unless ``cond``; ``msg`` is the text, or a function that
+    formats it (formatted on every call, the texts with shapes took a third of
+    an op's host time)."""
     if not cond:
-        raise exc(msg)
+        raise exc(msg() if callable(msg) else msg)
 
 
 def _on_gpu(name: str, t: torch.Tensor, dtype: torch.dtype | None = None, device=None) -> None:
@@ -66,7 +70,7 @@ def _on_gpu(name: str, t: torch.Tensor, dtype: torch.dtype | None = None, device
 
 
 def _cache_geometry(k_cache: torch.Tensor) -> tuple[int, int, int, int]:
-    _require(k_cache.dim() == 4, f"k_cache must be [num_blocks, num_kv_heads, block_size, head_dim], got {tuple(k_cache.shape)}")
+    _require(k_cache.dim() == 4, lambda: f"k_cache must be [num_blocks, num_kv_heads, block_size, head_dim], got {tuple(k_cache.shape)}")
     _require(k_cache.is_contiguous(), "k_cache must be contiguous")
     n, hkv, bs, d = k_cache.shape
     return n, hkv, bs, d
@@ -74,7 +78,7 @@ def _cache_geometry(k_cache: torch.Tensor) -> tuple[int, int, int, int]:
 
 def _tokens_view(x: torch.Tensor, name: str, hkv: int, d: int) -> torch.Tensor:
     _require(x.dim() == 3 and x.shape[1] == hkv and x.shape[2] == d,
-             f"{name} must be [num_tokens, {hkv}, {d}], got {tuple(x.shape)}")
+             lambda: f"{name} must be [num_tokens, {hkv}, {d}], got {tuple(x.shape)}")
     if x.stride(2) != 1:
         x = x.contiguous()
     return x
@@ -101,7 +105,7 @@ def quantize_kv_write_paged(k, v, k_cache, k_scale, v_cache, v_scale, slot_mappi
     v = _tokens_view(v, "v", hkv, d)
     t = k.shape[0]
     _require(v.shape[0] == t, "k and v token counts differ")
-    _require(slot_mapping.dim() == 1 and slot_mapping.shape[0] == t, f"slot_mapping must be [{t}]")
+    _require(slot_mapping.dim() == 1 and slot_mapping.shape[0] == t, lambda: f"slot_mapping must be [{t}]")
     if t == 0:
         return
     slot_mapping = slot_mapping.contiguous()
@@ -166,32 +170,29 @@ def _decode_prep(q, k_cache, block_table, context_lens, block_size, max_context_
     _on_gpu("block_table", block_table, torch.int32, dev)
     _on_gpu("context_lens", context_lens, torch.int32, dev)
     n, hkv, bs, d = _cache_geometry(k_cache)
-    _require(int(block_size) == bs, f"block_size {block_size} does not match the cache ({bs})")
-    squeeze = False
-    if q.dim() == 4:
-        _require(q.shape[2] == 1, f"decode q must be [B, Hq, 1, D], got {tuple(q.shape)}")
-        q3 = q[:, :, 0, :]
+    _require(int(block_size) == bs, lambda: f"block_size {block_size} does not match the cache ({bs})")
+    q_shape = tuple(q.shape)
+    if len(q_shape) == 4:
+        _require(q_shape[2] == 1, lambda: f"decode q must be [B, Hq, 1, D], got {q_shape}")
     else:
-        _require(q.dim() == 3, f"decode q must be [B, Hq, 1, D] or [B, Hq, D], got {tuple(q.shape)}")
-        q3 = q
-        squeeze = True
-    _require(q3.shape[2] == d, f"q head_dim {q3.shape[2]} != cache head_dim {d}")
-    if q3.stride(2) != 1:
-        q3 = q3.contiguous()
-    b, hq = q3.shape[0], q3.shape[1]
-    _require(block_table.dim() == 2 and block_table.shape[0] == b, f"block_table must be [{b}, max_blocks]")
+        _require(len(q_shape) == 3, lambda: f"decode q must be [B, Hq, 1, D] or [B, Hq, D], got {q_shape}")
+    b, hq = q_shape[:2]
+    _require(q_shape[-1] == d, lambda: f"q head_dim {q_shape[-1]} != cache head_dim {d}")
+    if q.stride(-1) != 1:
+        q = q.contiguous()
+    _require(block_table.dim() == 2 and block_table.shape[0] == b, lambda: f"block_table must be [{b}, max_blocks]")
     if block_table.stride(1) != 1:
         block_table = block_table.contiguous()
-    _require(context_lens.dim() == 1 and context_lens.shape[0] == b, f"context_lens must be [{b}]")
+    _require(context_lens.dim() == 1 and context_lens.shape[0] == b, lambda: f"context_lens must be [{b}]")
     context_lens = context_lens.contiguous()
     max_context_len = int(max_context_len)
     _require(max_context_len >= 0, "max_context_len must be >= 0")
     _require(max_context_len <= block_table.shape[1] * bs,
-             f"max_context_len {max_context_len} exceeds the block table capacity {block_table.shape[1] * bs}")
-    out = torch.empty((b, hq, 1, d) if not squeeze else (b, hq, d), dtype=torch.float16, device=dev)
+             lambda: f"max_context_len {max_context_len} exceeds the block table capacity {block_table.shape[1] * bs}")
+    out = torch.empty(q_shape, dtype=torch.float16, device=dev)
     ws_bytes = decode_workspace_bytes(b, hq, hkv, d, max_context_len)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-    return q3, block_table, context_lens, out, ws, ws_bytes, (n, hkv, bs, d, b, hq), max_context_len
+    return q, block_table, context_lens, out, ws, ws_bytes, (n, hkv, bs, d, b, hq), max_context_len
 
 
 def attn_paged_decode_cached(q, k_cache, k_scale, v_cache, v_scale, block_table, context_lens, block_size, *,
@@ -202,10 +203,10 @@ def attn_paged_decode_cached(q, k_cache, k_scale, v_cache, v_scale, block_table,
     ``q``: fp16 ``[B, Hq, 1, D]`` (a transpose view is fine).  Returns fp16
     ``[B, Hq, 1, D]``.  ``max_context_len`` only sizes the context split; every
     row is gated by its own ``context_lens`` entry."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_scale", k_scale, torch.float32, dev)
     _on_gpu("v_cache", v_cache, torch.int8, dev)
     _on_gpu("v_scale", v_scale, torch.float32, dev)
@@ -216,10 +217,10 @@ def attn_paged_decode_cached(q, k_cache, k_scale, v_cache, v_scale, block_table,
         return out
     lib = _lib.load()
     rc = lib.s8kv_decode_int8(
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(), n, bs,
         bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     _lib.check(rc, "attn_paged_decode_cached")
     return out
@@ -231,25 +232,25 @@ def attn_paged_decode_window(q, k_cache, k_scale, v_cache, v_scale, block_table,
     only its last ``window`` tokens, positions ``[max(0, L - window), L)``.
     The reference reads that window back dense and decodes per row
     (gqa_attention.py:191-196 with kv_cache.py:1233-1299)."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_scale", k_scale, torch.float32, dev)
     _on_gpu("v_cache", v_cache, torch.int8, dev)
     _on_gpu("v_scale", v_scale, torch.float32, dev)
     _require(v_cache.shape == k_cache.shape and v_cache.is_contiguous(), "v_cache must match k_cache")
     _require(tuple(k_scale.shape) == (n, hkv, bs) and k_scale.is_contiguous(), "k_scale must be [N, Hkv, bs]")
     _require(tuple(v_scale.shape) == (n, hkv, bs) and v_scale.is_contiguous(), "v_scale must be [N, Hkv, bs]")
-    _require(int(window) >= 1, f"window must be >= 1, got {window}")
+    _require(int(window) >= 1, lambda: f"window must be >= 1, got {window}")
     if b == 0:
         return out
     lib = _lib.load()
     rc = lib.s8kv_decode_window_int8(
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(), n, bs,
         bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, int(window), float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     _lib.check(rc, "attn_paged_decode_window")
     return out
@@ -284,12 +285,12 @@ def attn_paged_decode_plan(k_cache, block_table, context_lens, block_size, *, nu
     _on_gpu("context_lens", context_lens, torch.int32, dev)
     _require(layout in ("int8", "k8v3"), f"layout must be 'int8' or 'k8v3', got {layout!r}")
     n, hkv, bs, d = _cache_geometry(k_cache)
-    _require(int(block_size) == bs, f"block_size {block_size} does not match the cache ({bs})")
+    _require(int(block_size) == bs, lambda: f"block_size {block_size} does not match the cache ({bs})")
     _require(block_table.dim() == 2 and block_table.stride(1) == 1, "block_table must be a [B, max_blocks] tensor "
              "with unit stride on its last dim (the decode ops are then given the same tensor)")
     b = block_table.shape[0]
     _require(context_lens.dim() == 1 and context_lens.shape[0] == b and context_lens.is_contiguous(),
-             f"context_lens must be a contiguous [{b}] tensor")
+             lambda: f"context_lens must be a contiguous [{b}] tensor")
     lib = _lib.load()
     nbytes = int(lib.s8kv_decode_plan_size(hkv))
     if plan is None:
@@ -297,7 +298,7 @@ def attn_paged_decode_plan(k_cache, block_table, context_lens, block_size, *, nu
     else:
         _on_gpu("plan", plan, torch.int32, dev)
         _require(plan.is_contiguous() and plan.numel() * 4 >= nbytes,
-                 f"plan must be a contiguous int32 tensor of at least {nbytes // 4} elements")
+                 lambda: f"plan must be a contiguous int32 tensor of at least {nbytes // 4} elements")
         nbytes = plan.numel() * 4
     entry = lib.s8kv_decode_plan_adaptive if adaptive else lib.s8kv_decode_plan
     rc = entry(b, int(num_q_heads), hkv, d, 1 if layout == "k8v3" else 0, 1 if fused else 0, n, bs,
@@ -334,10 +335,10 @@ def attn_paged_decode_append(q, k_new, v_new, k_cache, k_scale, v_cache, v_scale
     launch then skips locating its work and issues its first loads at once.
     Same bytes and outputs as without it; a plan made for another geometry
     or other tensors is ignored."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_new", k_new, torch.float16, dev)
     _on_gpu("v_new", v_new, torch.float16, dev)
     _on_gpu("k_scale", k_scale, torch.float32, dev)
@@ -348,16 +349,16 @@ def attn_paged_decode_append(q, k_new, v_new, k_cache, k_scale, v_cache, v_scale
     _require(tuple(v_scale.shape) == (n, hkv, bs) and v_scale.is_contiguous(), "v_scale must be [N, Hkv, bs]")
     k_new = _tokens_view(k_new, "k_new", hkv, d)
     v_new = _tokens_view(v_new, "v_new", hkv, d)
-    _require(k_new.shape[0] == b and v_new.shape[0] == b, f"k_new and v_new must be [{b}, {hkv}, {d}]")
+    _require(k_new.shape[0] == b and v_new.shape[0] == b, lambda: f"k_new and v_new must be [{b}, {hkv}, {d}]")
     if b == 0:
         return out
     lib = _lib.load()
     args = (
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_new.data_ptr(), k_new.stride(0), k_new.stride(1), v_new.data_ptr(), v_new.stride(0), v_new.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(), n, bs,
         bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     if plan is None:
         rc = lib.s8kv_decode_append_int8(*args)
@@ -377,10 +378,10 @@ def attn_paged_decode_append_k8v3(q, k_new, v_new, k_cache, k_scale, v_packed, v
     does -- one launch for the pair the reference runs as its K8V3 write
     (kv_cache.py:587-626) and ``decode_attn_static`` (kv_cache.py:1167-1182).
     ``plan``: as for ``attn_paged_decode_append`` (made with layout "k8v3")."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_new", k_new, torch.float16, dev)
     _on_gpu("v_new", v_new, torch.float16, dev)
     _on_gpu("k_scale", k_scale, torch.float32, dev)
@@ -395,16 +396,16 @@ def attn_paged_decode_append_k8v3(q, k_new, v_new, k_cache, k_scale, v_packed, v
     _require(v_codebook.numel() == 8 and v_codebook.is_contiguous(), "v_codebook must hold 8 contiguous entries")
     k_new = _tokens_view(k_new, "k_new", hkv, d)
     v_new = _tokens_view(v_new, "v_new", hkv, d)
-    _require(k_new.shape[0] == b and v_new.shape[0] == b, f"k_new and v_new must be [{b}, {hkv}, {d}]")
+    _require(k_new.shape[0] == b and v_new.shape[0] == b, lambda: f"k_new and v_new must be [{b}, {hkv}, {d}]")
     if b == 0:
         return out
     lib = _lib.load()
     args = (
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_new.data_ptr(), k_new.stride(0), k_new.stride(1), v_new.data_ptr(), v_new.stride(0), v_new.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(), v_codebook.data_ptr(),
         lloyd_block, n, bs, bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     if plan is None:
         rc = lib.s8kv_decode_append_k8v3(*args)
@@ -419,10 +420,10 @@ def attn_paged_decode_k8v3(q, k_cache, k_scale, v_packed, v_norm, v_codebook, bl
     """Decode over the K8V3 cache with the 3-bit V dequantized in-kernel
     (``superl8.attn_paged_decode_k8v3``, kv_cache.py:1170-1182; positional
     order pinned by tests/test_k8v3_cache.py:179-186)."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_scale", k_scale, torch.float32, dev)
     _on_gpu("v_packed", v_packed, torch.int32, dev)
     _on_gpu("v_norm", v_norm, torch.float32, dev)
@@ -437,10 +438,10 @@ def attn_paged_decode_k8v3(q, k_cache, k_scale, v_packed, v_norm, v_codebook, bl
         return out
     lib = _lib.load()
     rc = lib.s8kv_decode_k8v3(
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(), v_codebook.data_ptr(),
         lloyd_block, n, bs, bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     _lib.check(rc, "attn_paged_decode_k8v3")
     return out
@@ -450,10 +451,10 @@ def attn_paged_decode_window_k8v3(q, k_cache, k_scale, v_packed, v_norm, v_codeb
                                   block_size, *, max_context_len, window, scale):
     """``attn_paged_decode_k8v3`` for a sliding-window layer: row b attends
     only its last ``window`` tokens (see ``attn_paged_decode_window``)."""
-    q3, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
+    q, bt, cl, out, ws, ws_bytes, geo, max_context_len = _decode_prep(
         q, k_cache, block_table, context_lens, block_size, max_context_len)
     n, hkv, bs, d, b, hq = geo
-    dev = q3.device
+    dev = q.device
     _on_gpu("k_scale", k_scale, torch.float32, dev)
     _on_gpu("v_packed", v_packed, torch.int32, dev)
     _on_gpu("v_norm", v_norm, torch.float32, dev)
@@ -464,15 +465,15 @@ def attn_paged_decode_window_k8v3(q, k_cache, k_scale, v_packed, v_norm, v_codeb
     lloyd_block = d // v_norm.shape[-1] if v_norm.dim() == 4 and v_norm.shape[-1] > 0 else 0
     _require(tuple(v_norm.shape[:3]) == (n, hkv, bs) and v_norm.is_contiguous(), "v_norm must be [N, Hkv, bs, D/128]")
     _require(v_codebook.numel() == 8 and v_codebook.is_contiguous(), "v_codebook must hold 8 contiguous entries")
-    _require(int(window) >= 1, f"window must be >= 1, got {window}")
+    _require(int(window) >= 1, lambda: f"window must be >= 1, got {window}")
     if b == 0:
         return out
     lib = _lib.load()
     rc = lib.s8kv_decode_window_k8v3(
-        q3.data_ptr(), b, hq, hkv, d, q3.stride(0), q3.stride(1),
+        q.data_ptr(), b, hq, hkv, d, q.stride(0), q.stride(1),
         k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(), v_codebook.data_ptr(),
         lloyd_block, n, bs, bt.data_ptr(), bt.stride(0), cl.data_ptr(), max_context_len, int(window), float(scale),
-        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q3),
+        out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q),
     )
     _lib.check(rc, "attn_paged_decode_window_k8v3")
     return out
@@ -489,33 +490,33 @@ def _verify_inputs(q, k_cache, k_scale, block_table, prefix_lens, block_size, qu
     _on_gpu("block_table", block_table, torch.int32, dev)
     _on_gpu("prefix_lens", prefix_lens, torch.int32, dev)
     n, hkv, bs, d = _cache_geometry(k_cache)
-    _require(int(block_size) == bs, f"block_size {block_size} does not match the cache ({bs})")
+    _require(int(block_size) == bs, lambda: f"block_size {block_size} does not match the cache ({bs})")
     _require(tuple(k_scale.shape) == (n, hkv, bs) and k_scale.is_contiguous(), "k_scale must be [N, Hkv, bs]")
-    _require(q.dim() == 4 and q.shape[3] == d, f"verify q must be [B, Hq, S, {d}], got {tuple(q.shape)}")
+    _require(q.dim() == 4 and q.shape[3] == d, lambda: f"verify q must be [B, Hq, S, {d}], got {tuple(q.shape)}")
     if q.stride(3) != 1:
         q = q.contiguous()
     b, hq, s_, _ = q.shape
-    _require(block_table.dim() == 2 and block_table.shape[0] == b, f"block_table must be [{b}, max_blocks]")
+    _require(block_table.dim() == 2 and block_table.shape[0] == b, lambda: f"block_table must be [{b}, max_blocks]")
     if block_table.stride(1) != 1:
         block_table = block_table.contiguous()
-    _require(prefix_lens.dim() == 1 and prefix_lens.shape[0] == b, f"prefix_lens must be [{b}]")
+    _require(prefix_lens.dim() == 1 and prefix_lens.shape[0] == b, lambda: f"prefix_lens must be [{b}]")
     prefix_lens = prefix_lens.contiguous()
     ql_ptr = None
     if query_lens is not None:
         _on_gpu("query_lens", query_lens, torch.int32, dev)
-        _require(query_lens.dim() == 1 and query_lens.shape[0] == b, f"query_lens must be [{b}]")
+        _require(query_lens.dim() == 1 and query_lens.shape[0] == b, lambda: f"query_lens must be [{b}]")
         query_lens = query_lens.contiguous()
         ql_ptr = query_lens.data_ptr()
     tm_ptr = None
     if tree_mask is not None:
         _on_gpu("tree_mask", tree_mask, torch.int64, dev)
-        _require(tuple(tree_mask.shape) == (b, s_), f"tree_mask must be int64 [{b}, {s_}]")
+        _require(tuple(tree_mask.shape) == (b, s_), lambda: f"tree_mask must be int64 [{b}, {s_}]")
         _require(s_ <= 64, "tree verify supports at most 64 drafts per row")
         tree_mask = tree_mask.contiguous()
         tm_ptr = tree_mask.data_ptr()
     max_context_len = int(max_context_len)
     _require(0 <= max_context_len <= block_table.shape[1] * bs,
-             f"max_context_len {max_context_len} exceeds the block table capacity {block_table.shape[1] * bs}")
+             lambda: f"max_context_len {max_context_len} exceeds the block table capacity {block_table.shape[1] * bs}")
     out = torch.empty((b, hq, s_, d), dtype=torch.float16, device=dev)
     # partials of a key-range split (few query blocks or very long rows)
     ws_bytes = int(_lib.load().s8kv_verify_workspace_size(b, hq, hkv, d, s_, max_context_len)) if b and s_ else 0
@@ -537,7 +538,7 @@ def _fresh_drafts(k_draft, v_draft, b, s_, hkv, d, dev):
     _require(k_draft is not None and v_draft is not None, "k_draft and v_draft go together")
     for name, t in (("k_draft", k_draft), ("v_draft", v_draft)):
         _on_gpu(name, t, torch.float16, dev)
-        _require(tuple(t.shape) == (b, s_, hkv, d), f"{name} must be [{b}, {s_}, {hkv}, {d}] (the layer's [B, S, Hkv, D])")
+        _require(tuple(t.shape) == (b, s_, hkv, d), lambda: f"{name} must be [{b}, {s_}, {hkv}, {d}] (the layer's [B, S, Hkv, D])")
     kr = rotate_rows(k_draft.float())  # contiguous fp32, rotated as the cache's K is
     vd = v_draft
     if vd.stride(3) != 1 or vd.data_ptr() % 16 or any(x % 8 for x in vd.stride()[:3]):
@@ -576,7 +577,7 @@ def attn_paged_verify(q, k_cache, k_scale, v_cache, v_scale, block_table, prefix
     lib = _lib.load()
     _require(window is not None or k_draft is None, "fresh drafts (k_draft / v_draft) need a window")
     if window is not None:
-        _require(int(window) >= 1, f"window must be >= 1, got {window}")
+        _require(int(window) >= 1, lambda: f"window must be >= 1, got {window}")
         alive, drafts = _fresh_drafts(k_draft, v_draft, out.shape[0], out.shape[2], hkv, d, dev)
         rc = lib.s8kv_verify_window_int8(
             *head, k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(), n, bs,
@@ -615,7 +616,7 @@ def attn_paged_verify_k8v3(q, k_cache, k_scale, v_packed, v_norm, v_codebook, bl
     lib = _lib.load()
     _require(window is not None or k_draft is None, "fresh drafts (k_draft / v_draft) need a window")
     if window is not None:
-        _require(int(window) >= 1, f"window must be >= 1, got {window}")
+        _require(int(window) >= 1, lambda: f"window must be >= 1, got {window}")
         alive, drafts = _fresh_drafts(k_draft, v_draft, out.shape[0], out.shape[2], hkv, d, dev)
         rc = lib.s8kv_verify_window_k8v3(
             *head, k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(),
@@ -649,7 +650,7 @@ def attn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
     _on_gpu("cu_seqlens_k", cu_seqlens_k, torch.int32, dev)
     _require(q.dim() == 3 and k.dim() == 3 and v.shape == k.shape and k.shape[2] == q.shape[2],
              "attn_varlen: q [Tq, Hq, D], k / v [Tk, Hkv, D]")
-    _require(window_left is None or int(window_left) >= 1, f"window_left must be >= 1, got {window_left}")
+    _require(window_left is None or int(window_left) >= 1, lambda: f"window_left must be >= 1, got {window_left}")
     tq, hq, d = q.shape
     hkv = k.shape[1]
     _require(cu_seqlens_q.dim() == 1 and cu_seqlens_q.shape == cu_seqlens_k.shape and cu_seqlens_q.numel() >= 1,
@@ -710,8 +711,8 @@ def copy_blocks(tensors: Sequence[torch.Tensor], src: Sequence[int] | torch.Tens
     ptrs, bbytes, lstrides = [], [], []
     for i, t in enumerate(tensors):
         _on_gpu(f"tensors[{i}]", t, None, dev)
-        _require(t.is_contiguous(), f"tensors[{i}] must be contiguous")
-        _require(t.shape[0] == nl and t.shape[1] == nb, f"tensors[{i}] must be [{nl}, {nb}, ...]")
+        _require(t.is_contiguous(), lambda: f"tensors[{i}] must be contiguous")
+        _require(t.shape[0] == nl and t.shape[1] == nb, lambda: f"tensors[{i}] must be [{nl}, {nb}, ...]")
         per_block = t[0, 0].numel() * t.element_size()
         ptrs.append(t.data_ptr())
         bbytes.append(per_block)
@@ -725,7 +726,7 @@ def copy_blocks(tensors: Sequence[torch.Tensor], src: Sequence[int] | torch.Tens
     else:
         src_l, dst_l = [int(x) for x in src], [int(x) for x in dst]
         _require(len(src_l) == len(dst_l), "src and dst differ in length")
-        _require(all(0 <= x < nb for x in src_l + dst_l), f"block ids must be in [0, {nb})")
+        _require(all(0 <= x < nb for x in src_l + dst_l), lambda: f"block ids must be in [0, {nb})")
         _require(not (set(src_l) & set(dst_l)), "source and destination blocks overlap")
         _require(len(set(dst_l)) == len(dst_l), "destination blocks repeat")
         if not src_l:
@@ -754,7 +755,7 @@ _ROT_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 def _rows_view(x: torch.Tensor, name: str) -> torch.Tensor:
     """``x`` as ``[rows, D]`` with a unit stride on D (copies when the leading
     axes cannot be flattened into one row stride)."""
-    _require(x.dim() >= 1, f"{name} must have at least one dimension")
+    _require(x.dim() >= 1, lambda: f"{name} must have at least one dimension")
     d = x.shape[-1]
     x2 = x.reshape(-1, d)
     if x2.numel() and (x2.stride(1) != 1 or (x2.shape[0] > 1 and x2.stride(0) < d)):
@@ -768,7 +769,7 @@ def rotate_rows(x: torch.Tensor) -> torch.Tensor:
     dtype), the rotation the append applies to K.  fp16, bf16 or fp32; D in
     {32, 64, 128, 256}.  Returns a new tensor of x's shape and dtype."""
     _on_gpu("x", x)
-    _require(x.dtype in _ROT_DTYPES, f"rotate_last: dtype {x.dtype} not in fp16 / bf16 / fp32", TypeError)
+    _require(x.dtype in _ROT_DTYPES, lambda: f"rotate_last: dtype {x.dtype} not in fp16 / bf16 / fp32", TypeError)
     x2 = _rows_view(x, "x")
     d = x.shape[-1]
     out = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
@@ -824,7 +825,7 @@ def pack_codes3(codes: torch.Tensor) -> torch.Tensor:
     _on_gpu("codes", codes, torch.uint8)
     c2 = codes.reshape(-1, codes.shape[-1]).contiguous()
     d = codes.shape[-1]
-    _require(d % 32 == 0, f"pack_indices_lowbit: last dimension {d} is not a multiple of 32")
+    _require(d % 32 == 0, lambda: f"pack_indices_lowbit: last dimension {d} is not a multiple of 32")
     words = torch.empty((c2.shape[0], d * 3 // 32), dtype=torch.int32, device=codes.device)
     if c2.numel():
         lib = _lib.load()
@@ -839,7 +840,7 @@ def unpack_codes3(words: torch.Tensor, d: int) -> torch.Tensor:
     _on_gpu("words", words, torch.int32)
     d = int(d)
     _require(d > 0 and d % 32 == 0 and words.shape[-1] == d * 3 // 32,
-             f"unpack_indices_lowbit: {words.shape[-1]} words per row do not hold {d} 3-bit codes")
+             lambda: f"unpack_indices_lowbit: {words.shape[-1]} words per row do not hold {d} 3-bit codes")
     w2 = words.reshape(-1, words.shape[-1]).contiguous()
     codes = torch.empty((w2.shape[0], d), dtype=torch.uint8, device=words.device)
     if w2.numel():
@@ -855,7 +856,7 @@ def unpack_codes3(words: torch.Tensor, d: int) -> torch.Tensor:
 
 
 def _q_rows(q: torch.Tensor, num_q_heads: int) -> torch.Tensor:
-    _require(q.dtype in (torch.float16, torch.float32), f"q must be fp16 or fp32, got {q.dtype}", TypeError)
+    _require(q.dtype in (torch.float16, torch.float32), lambda: f"q must be fp16 or fp32, got {q.dtype}", TypeError)
     q2 = q.reshape(num_q_heads, -1)
     if q2.stride(1) != 1:
         q2 = q2.contiguous()
@@ -885,11 +886,11 @@ def snapkv_scores(q: torch.Tensor, k: torch.Tensor, num_heads: int, num_kv_heads
     if k.dim() == 4:
         _require(k.shape[0] == 1, "k_full [1, Hkv, S, D] expected")
         k = k[0]
-    _require(k.dim() == 3 and k.shape[0] == num_kv_heads, f"k_full must be [{num_kv_heads}, S, D]")
-    _require(k.dtype in (torch.float16, torch.float32), f"k_full must be fp16 or fp32, got {k.dtype}", TypeError)
+    _require(k.dim() == 3 and k.shape[0] == num_kv_heads, lambda: f"k_full must be [{num_kv_heads}, S, D]")
+    _require(k.dtype in (torch.float16, torch.float32), lambda: f"k_full must be fp16 or fp32, got {k.dtype}", TypeError)
     d = k.shape[2]
     q2 = _q_rows(q, num_heads)
-    _require(q2.shape[1] == d, f"q_last head_dim {q2.shape[1]} != k_full head_dim {d}")
+    _require(q2.shape[1] == d, lambda: f"q_last head_dim {q2.shape[1]} != k_full head_dim {d}")
     if k.stride(2) != 1:
         k = k.contiguous()
     sc = 1.0 / math.sqrt(d) if scale is None else float(scale)
@@ -914,10 +915,10 @@ def snapkv_scores_paged(q: torch.Tensor, k_cache: torch.Tensor, k_scale: torch.T
     length = int(length)
     need = -(-length // bs)
     blocks = [int(b) for b in blocks]
-    _require(len(blocks) >= need, f"{len(blocks)} blocks cannot hold {length} tokens")
-    _require(all(0 <= b < n for b in blocks[:need]), f"block ids must be in [0, {n})")
+    _require(len(blocks) >= need, lambda: f"{len(blocks)} blocks cannot hold {length} tokens")
+    _require(all(0 <= b < n for b in blocks[:need]), lambda: f"block ids must be in [0, {n})")
     q2 = _q_rows(q, num_heads)
-    _require(q2.shape[1] == d, f"q_last head_dim {q2.shape[1]} != cache head_dim {d}")
+    _require(q2.shape[1] == d, lambda: f"q_last head_dim {q2.shape[1]} != cache head_dim {d}")
     row = torch.tensor(blocks[:max(need, 1)], dtype=torch.int32).to(dev)
     sc = 1.0 / math.sqrt(d) if scale is None else float(scale)
     return _snapkv_run(length, num_heads, dev, lambda lib, out, ws, nb: lib.s8kv_snapkv_scores_paged(
@@ -939,14 +940,14 @@ def gather_slots(tensors: Sequence[torch.Tensor], src_slots: Sequence[int], dst_
     _on_gpu("tensors[0]", t0)
     dev = t0.device
     nl, nb, hkv, bs = t0.shape[:4]
-    _require(int(block_size) == bs, f"block_size {block_size} does not match the cache ({bs})")
-    _require(all(0 <= x < nb * bs for x in src_l + dst_l), f"slots must be in [0, {nb * bs})")
+    _require(int(block_size) == bs, lambda: f"block_size {block_size} does not match the cache ({bs})")
+    _require(all(0 <= x < nb * bs for x in src_l + dst_l), lambda: f"slots must be in [0, {nb * bs})")
     _require(not (set(src_l) & set(dst_l)), "source and destination slots overlap")
     ptrs, rbytes, lstrides = [], [], []
     for i, t in enumerate(tensors):
         _on_gpu(f"tensors[{i}]", t, None, dev)
         _require(t.is_contiguous() and tuple(t.shape[:4]) == (nl, nb, hkv, bs),
-                 f"tensors[{i}] must be contiguous [{nl}, {nb}, {hkv}, {bs}, ...]")
+                 lambda: f"tensors[{i}] must be contiguous [{nl}, {nb}, {hkv}, {bs}, ...]")
         ptrs.append(t.data_ptr())
         rbytes.append(t[0, 0, 0, 0].numel() * t.element_size())
         lstrides.append(t.stride(0) * t.element_size())
