@@ -2004,7 +2004,11 @@ struct FreshDrafts {
 //    is the common case -- so units are split until about that many exist,
 //    down to kMinSplitKeys keys per split (512: a 32K-key batch-1 tree verify
 //    at 8 KV heads fills all 512 slots, 4-5 % faster than 32 splits of 1024
-//    keys; a second round of splits is slower again);
+//    keys; a second round of splits is slower again), and where even one per
+//    CU is not reached, down to kFewUnitKeys where that makes 3 splits or more
+//    (2 lose up to 15 % to the combine; us a call at 512 and 128 keys: one
+//    98-query chunk behind 662 keys, head_dim 256, 2 heads 73 / 33; 2 trees of
+//    36 over 1,242, head_dim 64, 4 heads 32 / 19; 3 of 898, 2 heads 34 / 20);
 //  * rows of different lengths: with whole rows (or halves of each) the
 //    longest one runs alone at the end.  Splits of at least kMinSplitKeys keys,
 //    and 32 keys per query row (a split writes and the combine reads 1 KB a
@@ -2021,6 +2025,7 @@ struct FreshDrafts {
 // the rounding of its fp32 sums.  s8kv_verify_set_splits overrides the count
 // (diagnostics).
 constexpr int kMinSplitKeys = 512;
+constexpr int kFewUnitKeys = 128;
 constexpr int kBalanceRounds = 8;
 constexpr int kMaxSplitKeys = 1 << 20;
 constexpr int kMaxSplits = 1024;
@@ -2035,12 +2040,14 @@ static int verify_plan_splits(int batch, int num_kv_heads, int n_qblocks, int ke
   int64_t s = natural < resident ? (resident + natural - 1) / natural : 1;
   const int64_t fill = s;
   s = std::min<int64_t>(s, std::max(1, keys / kMinSplitKeys));
+  const int64_t few = std::min<int64_t>(device_cus() / natural, keys / kFewUnitKeys);
+  if (few >= 3) s = std::max(s, few);
   if (batch > 1) {
     const int64_t least = std::max(kMinSplitKeys, 32 * std::min(rows, rows_wg));
     s = std::max(s, units(kBalanceRounds * resident, least) / fill * fill);
   }
   if (wide && verify::wide_narrow(rows))
-    s = std::max({units(device_cus(), 128), units(2 * device_cus(), 512), units(6 * device_cus(), 1024)});
+    s = std::max({units(device_cus(), kFewUnitKeys), units(2 * device_cus(), 512), units(6 * device_cus(), 1024)});
   s = std::max<int64_t>(s, ((int64_t)keys + kMaxSplitKeys - 1) / kMaxSplitKeys);
   const int forced = g_verify_splits.load();
   if (forced > 0) s = forced;
