@@ -47,6 +47,12 @@ constexpr float kMaxSlack = 8.0f;
 // score (-inf) and never NaN, with no test per score; any real score exceeds
 // it by more than kMaxSlack + esh, which makes the first visible tile rescale (by 0).
 constexpr float kMaxInit = -1.0e30f;
+// Staged V scales of the 32-row kernel: finite ones are capped at kScaleCap, and
+// kBadScale stands for a non-finite one.  It is above every bound that
+// WeightShift::raise sets for the others (2^101 at most), so each tile holding
+// one takes the rescale branch, where the rows that see it get their NaN.
+constexpr float kScaleCap = 0x1p100f;
+constexpr float kBadScale = 0x1p110f;
 
 template <int D, bool K8V3>
 struct Cfg {
@@ -1122,14 +1128,16 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       }
     }
   };
-  // a V scale is staged finite (NaN and inf -> 2^100): the weight of a hidden
-  // key, exp2(-inf) * scale, is then 0 whatever was stored there (clamped
-  // here, where the load is consumed, not where it is issued); a fresh
-  // draft's K and V scales are 1
+  // a V scale is staged finite (above 2^100: that; NaN and +-inf: kBadScale),
+  // so the weight of a hidden key, exp2(-inf) * scale, is 0 whatever was
+  // stored there; weights() gives the rows that see a kBadScale key their NaN
+  // (clamped here, where the load is consumed, not where it is issued); a
+  // fresh draft's K and V scales are 1
   auto store_scale = [&](int buf, int base, int tt, int side, float v) {  // side 0: K, 1 + n: V block n
     float* sb = reinterpret_cast<float*>(smem + buf * C::BUF + C::KBYTES + C::VBYTES);
     const bool k_side = side == 0;
-    sb[side * kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : k_side ? v : fminf(v, 0x1p100f);
+    if (!k_side) v = __builtin_isfinite(v) ? fminf(v, kScaleCap) : kBadScale;
+    sb[side * kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : v;
   };
 
   // ---- one 32-key tile from LDS buffer `buf`: scores, weights, PV ----
@@ -1215,8 +1223,9 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       // the running max rises to the tile's (from the products, exactly),
       // l and the accumulators are rescaled, the scores re-referenced
       int d = 0;
-      if (__builtin_amdgcn_ballot_w64(vp > ws.vbound()) != 0) {
-        float vmx = fmaxf(vp, shfl_xor_f(vp, 1));
+      const float vf = vp != kBadScale ? vp : 0.0f;  // (NaN for the rows that see it, whatever the shift)
+      if (__builtin_amdgcn_ballot_w64(vf > ws.vbound()) != 0) {
+        float vmx = fmaxf(vf, shfl_xor_f(vf, 1));
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 2));
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 4));
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 8));
@@ -1235,6 +1244,21 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       m_ref = m_new;
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) y[rr] = y[rr] != kNegInf ? __builtin_fmaf(sc[rr], kscale(rr), -m_new) : kNegInf;
+      // a visible non-finite V scale: NaN in the dims it scales, as its product
+      // with any weight (the kernel's hi + lo split of inf is inf - inf) gives
+      if (!DENSE && __builtin_amdgcn_ballot_w64(vp == kBadScale) != 0) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          float bad = 0.0f;
+#pragma unroll
+          for (int rr = 0; rr < 16; ++rr)
+            if (row_live && y[rr] != kNegInf && sb[(1 + nb) * kTile + 8 * (rr >> 2) + 4 * hf + (rr & 3)] == kBadScale)
+              bad = __builtin_nanf("");
+          bad = sum_x32(bad);
+#pragma unroll
+          for (int n = nb * NT / NB; n < (nb + 1) * NT / NB; ++n) acc[n] += bad;
+        }
+      }
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
