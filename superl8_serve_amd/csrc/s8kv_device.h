@@ -26,8 +26,11 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 // ---------------------------------------------------------------------------
 // Buffer resources: every bulk cache access goes through a buffer descriptor
-// whose num_records is the tensor's byte size, so an index that escapes the
-// tensor reads zeros instead of faulting.
+// whose num_records is the tensor's byte size.  The range check covers the
+// per-lane offset: an index that escapes the tensor through it reads zeros
+// instead of faulting (the verify kernels' block ids).  A scalar offset (`soff`)
+// is not covered: the decode kernels, whose tiles start at one, rely on valid
+// block ids in the entries that a row's context length reaches.
 // ---------------------------------------------------------------------------
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 

@@ -1355,9 +1355,9 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
           float s[1 + NB];
         } R;
         auto load_tile = [&](int base) {
-          // one block holds the tile (bs >= 32): scalar offset of its first row
-          // (rows past the last key are read too, and masked; not their
-          // scales); else a row per lane
+          // one block holds the tile (bs >= 32): from a scalar first row (rows
+          // past the last key are read too, and masked; not their scales);
+          // else a row per lane
           const int lim = u1 - 1 - base;  // the last key of the range, from the tile's first
           const bool one = bs_log2 >= 5;
           auto row_of = [&](int tt) -> uint32_t {
@@ -1367,9 +1367,9 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
           const uint32_t row = one ? (uint32_t)__builtin_amdgcn_readfirstlane((int)row_of(0)) : 0u;
           uint32_t at[C::NCH];
           const int tk = lane & (kTile - 1);
-          uint32_t scale_at = (uint32_t)min(tk, lim);
+          uint32_t scale_at = row + (uint32_t)min(tk, lim);
 #pragma unroll
-          for (int i = 0; i < C::NCH; ++i) at[i] = (uint32_t)((lane + 64 * i) / PARTS);
+          for (int i = 0; i < C::NCH; ++i) at[i] = row + (uint32_t)((lane + 64 * i) / PARTS);
           if (!one) {
             scale_at = row_of(tk);
 #pragma unroll
@@ -1378,22 +1378,20 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
 #pragma unroll
           for (int i = 0; i < C::NCH; ++i) {
             const uint32_t part = (uint32_t)((lane + 64 * i) % PARTS);
-            R.k[i] = bload128<kNT>(kc, at[i] * (uint32_t)D + part * 16u, row * (uint32_t)D);
+            R.k[i] = bload128<kNT>(kc, at[i] * (uint32_t)D + part * 16u);
             if constexpr (K8V3) {
-              const u32x3_t w = bload96<kNT>(vc, at[i] * (uint32_t)(C::WORDS * 4) + (part >> 1) * 12u,
-                                             row * (uint32_t)(C::WORDS * 4));
+              const u32x3_t w = bload96<kNT>(vc, at[i] * (uint32_t)(C::WORDS * 4) + (part >> 1) * 12u);
               R.v[i].x = w.x;
               R.v[i].y = w.y;
               R.v[i].z = w.z;
             } else {
-              R.v[i] = bload128<kNT>(vc, at[i] * (uint32_t)D + part * 16u, row * (uint32_t)D);
+              R.v[i] = bload128<kNT>(vc, at[i] * (uint32_t)D + part * 16u);
             }
           }
           // (by both halves of the wave: see the 4-wave loop)
-          R.s[0] = __builtin_bit_cast(float, bload32(ks, scale_at * 4u, row * 4u));
+          R.s[0] = __builtin_bit_cast(float, bload32(ks, scale_at * 4u));
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            R.s[1 + nb] = __builtin_bit_cast(float, bload32(vs, (scale_at * NB + nb) * 4u, row * (NB * 4u)));
+          for (int nb = 0; nb < NB; ++nb) R.s[1 + nb] = __builtin_bit_cast(float, bload32(vs, (scale_at * NB + nb) * 4u));
         };
         auto store_tile = [&](int base) {
 #pragma unroll
@@ -1530,21 +1528,21 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
         } else {
           const int lim = min(u1 - 1 - base, kTile - 1);  // the tile's last key
           const int key = min(tt, lim);
-          // one block: scalar offsets of its first row (rows past the last key
-          // are read too, and masked; not their scales); else a row per lane.
+          // one block: from a scalar first row (rows past the last key are
+          // read too, and masked; not their scales); else a row per lane.  The
+          // row is part of the lanes' offsets, which the range check covers.
           // (offsets are chosen and not loads: a choice of loads waits for those in flight)
           const uint32_t bid = (uint32_t)__builtin_amdgcn_readfirstlane(R.bid);
-          uint32_t row = ((bid * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)base & bsm);
-          uint32_t off = lane_off, soff = (uint32_t)key * 4u;
+          const uint32_t row = ((bid * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)base & bsm);
+          uint32_t off = lane_off + row * row_bytes, soff = ((uint32_t)key + row) * 4u;
           if (bs_log2 < 5) {
-            row = 0;
             const uint32_t lane_row =
                 (((uint32_t)R.bid * hkv + (uint32_t)h) << bs_log2) + ((uint32_t)(base + key) & bsm);
-            off += (lane_row - (uint32_t)tt) * row_bytes;
+            off = lane_off + (lane_row - (uint32_t)tt) * row_bytes;
             soff = lane_row * 4u;
           }
-          R.s = __builtin_bit_cast(float, bload32(rs, soff, row * 4u));
-          R.d[0] = bload128(rc, off, row * row_bytes);
+          R.s = __builtin_bit_cast(float, bload32(rs, soff));
+          R.d[0] = bload128(rc, off);
           R.bid = block_id(next + 2 * kTile);
         }
       };

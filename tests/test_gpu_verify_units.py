@@ -117,6 +117,38 @@ def test_more_than_128_rows(kind, d, bs, nq, tree, window):
            query_lens=[nq, nq, 1, nq - 1, nq, 9, nq, nq, 0], window=window, tree=tree)
 
 
+@pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
+@pytest.mark.parametrize("nq", [5, 20, 50])  # of 4 heads: one 32-row wave, a 128-row workgroup, more
+@pytest.mark.parametrize("bs", [16, 32, 64])
+def test_block_id_past_the_pool_reads_zeros(kind, d, nq, bs):
+    """The pool is the front of a larger allocation: a table entry naming the
+    block after the pool's last gives the outputs of an all-zero block, not of
+    what is stored there."""
+    prefix = np.array([300, 150])
+    case = make_case(90 + d, 2, 8, 2, d, bs, prefix + nq)
+    n = case.num_blocks
+    whole = alloc(kind, n + 3, 2, bs, d)
+    append(kind, t(case.k), t(case.v), whole, t(case.slots))
+    for x in whole:
+        x[n:] = 3  # (past the pool below)
+    spare = next(i for i in range(n) if i not in set(case.block_table.ravel()))
+    cache = [x[:n] for x in whole]
+    for x in cache:
+        x[spare] = 0
+    q = t(np.random.default_rng(91).standard_normal((2, 8, nq, d)).astype(np.float16))
+    fn = ops.attn_paged_verify if kind == "int8" else ops.attn_paged_verify_k8v3
+    extra = () if kind == "int8" else (t(CODEBOOK),)
+    outs = []
+    for block in (spare, n):
+        table = case.block_table.copy()
+        table[0, 1] = table[1, 0] = block
+        out = fn(q, *cache, *extra, t(table), t(prefix.astype(np.int32)), bs,
+                 max_context_len=int(case.lens.max()), scale=case.scale)
+        torch.cuda.synchronize()
+        outs.append(to_np(out))
+    assert np.isfinite(outs[0]).all() and np.array_equal(*outs)
+
+
 def test_workspace_counts_the_split():
     """The workspace query plans the ragged batch's split too, and a call
     without a workspace runs unsplit."""
