@@ -47,12 +47,12 @@ constexpr float kMaxSlack = 8.0f;
 // score (-inf) and never NaN, with no test per score; any real score exceeds
 // it by more than kMaxSlack + esh, which makes the first visible tile rescale (by 0).
 constexpr float kMaxInit = -1.0e30f;
-// Staged V scales of the 32-row kernel: finite ones are capped at kScaleCap, and
-// kBadScale stands for a non-finite one.  It is above every bound that
-// WeightShift::raise sets for the others (2^101 at most), so each tile holding
-// one takes the rescale branch, where the rows that see it get their NaN.
-constexpr float kScaleCap = 0x1p100f;
-constexpr float kBadScale = 0x1p110f;
+// What the 32-row kernel stages for a non-finite V scale.  It is above every
+// bound that WeightShift::raise sets for a scale of at most kScaleCap, so each
+// tile holding one takes the rescale branch, where the rows that see it get
+// their NaN.
+constexpr float kBadScale = 0x1.fffffep127f;
+constexpr float kScaleCap = 0x1p126f;
 
 template <int D, bool K8V3>
 struct Cfg {
@@ -1128,15 +1128,15 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       }
     }
   };
-  // a V scale is staged finite (above 2^100: that; NaN and +-inf: kBadScale),
-  // so the weight of a hidden key, exp2(-inf) * scale, is 0 whatever was
-  // stored there; weights() gives the rows that see a kBadScale key their NaN
-  // (clamped here, where the load is consumed, not where it is issued); a
-  // fresh draft's K and V scales are 1
+  // a V scale is staged finite (NaN and +-inf: kBadScale), so the weight of a
+  // hidden key, exp2(-inf) * scale, is 0 whatever was stored there; weights()
+  // gives the rows that see a kBadScale key their NaN (replaced here, where
+  // the load is consumed, not where it is issued); a fresh draft's K and V
+  // scales are 1
   auto store_scale = [&](int buf, int base, int tt, int side, float v) {  // side 0: K, 1 + n: V block n
     float* sb = reinterpret_cast<float*>(smem + buf * C::BUF + C::KBYTES + C::VBYTES);
     const bool k_side = side == 0;
-    if (!k_side) v = __builtin_isfinite(v) ? fminf(v, kScaleCap) : kBadScale;
+    v = k_side || __builtin_isfinite(v) ? v : kBadScale;
     sb[side * kTile + tt] = fresh_draft(base, tt) >= 0 ? 1.0f : v;
   };
 
@@ -1229,7 +1229,7 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 2));
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 4));
         vmx = fmaxf(vmx, shfl_xor_f(vmx, 8));
-        d = ws.raise(max_x16(vmx), kMaxSlack);
+        d = ws.raise(fminf(max_x16(vmx), kScaleCap), kMaxSlack);
       }
       m_ref -= (float)d;
       float mt = kNegInf;
