@@ -402,6 +402,22 @@ def test_adaptive_plan_falls_back_on_new_lengths():
     _same(step.run(plan), step.run(None), "adaptive plan after a length rewrite")
 
 
+@pytest.mark.parametrize("lens", [[30011], [2900, 2100, 1700, 2600], [40000, 1]])
+def test_adaptive_plan_keeps_the_least_slice(lens):
+    """Few rows: the fixed split leaves columns without a slice so that no row
+    is cut finer than pays, and adapting does not hand them one."""
+    step = _Step(make_case(5656, len(lens), 32, 8, 128, 256, lens), "int8")
+    ref = step.run(None)
+    plan = step.plan(adaptive=True)
+    fixed = _adaptive_area(plan, 8)[1]
+    assert (np.diff(fixed) == 0).any()
+    for k in range(8):
+        _check_close(step.run(plan), ref, f"adaptive step {k}")
+        step.plan(adaptive=True, plan=plan)
+        bd = _adaptive_area(plan, 8)[1]
+        assert (np.diff(bd) > 0).sum() <= (np.diff(fixed) > 0).sum(), f"step {k}: more slices than the fixed split"
+
+
 def test_adaptive_plan_graph_replays():
     """The adaptive plan launch and three layers' planned decode launches in
     one graph, replayed: the bounds adapt from replay to replay, every replay
