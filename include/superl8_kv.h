@@ -295,8 +295,8 @@ int s8kv_decode_window_k8v3(const void* q, int batch, int num_q_heads, int num_k
  * for a tree it generalizes the chain to an ancestor mask.
  *
  * q: fp16 [batch, num_q_heads, max_queries, head_dim] with element strides
- * q_stride_b, q_stride_h, q_stride_s (head_dim contiguous).  Row b has
- * prefix_lens[b] prefix keys followed by query_lens[b] draft keys (or
+ * q_stride_b, q_stride_h, q_stride_s (head_dim contiguous, rows of any
+ * alignment; out 8-byte aligned).  Row b has prefix_lens[b] prefix keys followed by query_lens[b] draft keys (or
  * max_queries when query_lens is NULL), already appended to the cache at
  * positions prefix_lens[b] .. prefix_lens[b]+n-1.  Query s of row b attends
  * every prefix key plus draft key i when i <= s (tree_mask NULL: chain /

@@ -992,7 +992,9 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
                          (int64_t)(row_live ? pos : 0) * a.q_stride_s + hf * HALF;
 #pragma unroll
     for (int i = 0; i < HALF; i += 8) {
-      const half8_t v = *reinterpret_cast<const half8_t*>(qp + i);
+      // (rows of any alignment: a view may start inside one)
+      typedef _Float16 any_half8_t __attribute__((ext_vector_type(8), aligned(2)));
+      const half8_t v = *reinterpret_cast<const any_half8_t*>(qp + i);
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[i + e] = row_live ? (float)v[e] : 0.0f;
     }

@@ -119,6 +119,26 @@ def test_more_than_128_rows(kind, d, bs, nq, tree, window):
 
 @pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
 @pytest.mark.parametrize("nq", [5, 20, 50])  # of 4 heads: one 32-row wave, a 128-row workgroup, more
+@pytest.mark.parametrize("offset,pitch", [(1, 3), (4, 12), (8, 8)])
+def test_q_rows_of_any_alignment(kind, d, nq, offset, pitch):
+    """q as a view that starts `offset` elements into rows of d + `pitch`: the
+    same bits as the aligned copy."""
+    prefix = np.array([300, 150])
+    case = make_case(95 + d, 2, 8, 2, d, 32, prefix + nq)
+    cache = alloc(kind, case.num_blocks, 2, 32, d)
+    append(kind, t(case.k), t(case.v), cache, t(case.slots))
+    rows = t(np.random.default_rng(96).standard_normal((2, nq, 8, d + pitch)).astype(np.float16))
+    view = rows[..., offset:offset + d].transpose(1, 2)
+    fn = ops.attn_paged_verify if kind == "int8" else ops.attn_paged_verify_k8v3
+    extra = () if kind == "int8" else (t(CODEBOOK),)
+    outs = [fn(q, *cache, *extra, t(case.block_table), t(prefix.astype(np.int32)), 32,
+               max_context_len=int(case.lens.max()), scale=case.scale) for q in (view, view.contiguous())]
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+
+
+@pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
+@pytest.mark.parametrize("nq", [5, 20, 50])  # of 4 heads: one 32-row wave, a 128-row workgroup, more
 @pytest.mark.parametrize("bs", [16, 32, 64])
 def test_block_id_past_the_pool_reads_zeros(kind, d, nq, bs):
     """The pool is the front of a larger allocation: a table entry naming the
