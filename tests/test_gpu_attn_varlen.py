@@ -132,6 +132,25 @@ def test_attn_varlen_unaligned_q(window_left):
     _close(out.float().cpu().numpy(), ref, f"unaligned q, window {window_left}")
 
 
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("hkv", [2, 8])
+@pytest.mark.parametrize("window_left,causal", [(None, True), (50, True), (None, False)])
+def test_attn_varlen_unaligned_q_head_dims(d, hkv, window_left, causal):
+    """The 16-row kernel at its other head_dims: q rows 4 elements into wider
+    ones, sequences of one to several blocks, and one with more queries than keys."""
+    qlens, klens = [120, 9, 33, 300], [200, 9, 20, 300]
+    q, k, v, cu_q, cu_k = _case(790 + d, 8, hkv, d, qlens, klens)
+    qbig = np.zeros((q.shape[0], 8, d + 8), np.float16)
+    qbig[:, :, 4:4 + d] = q
+    qv = _t(qbig)[:, :, 4:4 + d]
+    assert qv.data_ptr() % 16 != 0
+    out = ops.attn_varlen(qv, _t(k), _t(v), _t(cu_q), _t(cu_k), 300, 300, causal=causal, scale=d ** -0.5,
+                          window_left=window_left)
+    torch.cuda.synchronize()
+    ref = O.dense_varlen_attention(q, k, v, cu_q, cu_k, d ** -0.5, causal, window_left=window_left)
+    _close(out.float().cpu().numpy(), ref, f"unaligned q, D={d}, window {window_left}")
+
+
 def test_attn_varlen_wide_window_equals_plain_causal():
     q, k, v, cu_q, cu_k = _case(761, 8, 2, 128, [200, 50], [200, 90])
     args = (_t(q), _t(k), _t(v), _t(cu_q), _t(cu_k), 200, 200)
