@@ -1,8 +1,15 @@
 // Multi-query verify attention over the paged int8 or K8V3 cache: tree verify (each
 // draft query sees the prefix plus its ancestors in the draft tree) and
-// chunked prefill / chain verify (query s sees the prefix plus drafts 0..s).
+// chunked prefill / chain verify (query s sees the prefix plus drafts 0..s);
+// and dense prefill attention over fresh fp16 K and V.
 //
-// Layout of the work: a workgroup of W waves (4; 8 for K8V3) owns 16 * W * RG
+// Two kernels.  verify_wide_kernel (32 query rows per wave, described there)
+// serves the calls whose tensors fit 32-bit offsets and whose dense q and
+// output rows are aligned.  verify_kernel (16 rows per wave) serves the rest:
+// pools past 4 GiB a layer, whose tiles are loaded through descriptors rebased
+// to each tile, and dense calls with unaligned rows.
+//
+// Layout of verify_kernel's work: a workgroup of W waves (4; 8 for K8V3) owns 16 * W * RG
 // query rows of one (sequence, KV head) pair -- row r is query position r / G of q head
 // h*G + r % G -- and streams the pair's keys in 32-key tiles.  Each tile's K
 // and V rows are loaded once per workgroup, converted int8 -> fp16 (exact) on
@@ -98,8 +105,8 @@ struct VerifyArgs {
   const float* v_scale;       // int8 V scales, or K8V3 block norms
   const float* v_codebook;    // K8V3: fp32 [8]
   uint32_t kc_bytes, ks_bytes, vc_bytes, vs_bytes;
-  // the tensors' full sizes; verify_kernel<.., BIG> (a tensor past 4 GiB,
-  // block_size >= 32) loads each tile through descriptors rebased to it
+  // the tensors' full sizes; verify_kernel (a tensor past 4 GiB, block_size
+  // >= 32) loads each tile through descriptors rebased to it
   uint64_t kc_total, ks_total, vc_total, vs_total;
   int big;
   const int32_t* block_table;
@@ -178,10 +185,9 @@ __device__ __forceinline__ void split_range(const VerifyArgs& a, int sp, int end
 // transpose-read rows (keys 4g..4g+3 and 16+4g..16+4g+3) are rows 8g..8g+7.
 __device__ __forceinline__ int vrow_of(int tt) { return 8 * ((tt & 15) >> 2) + 4 * (tt >> 4) + (tt & 3); }
 
-template <int D, bool K8V3, bool WIN = false, bool DENSE = false, bool BIG = false>
+template <int D, bool K8V3, bool WIN = false, bool DENSE = false>
 __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kernel(VerifyArgs a) {
   static_assert(!DENSE || !K8V3, "dense inputs: fp16 K / V");
-  static_assert(!DENSE || !BIG, "dense inputs are not paged");
   using C = Cfg<D, K8V3>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int* bt_lds = reinterpret_cast<int*>(smem + 2 * C::BUF);
@@ -310,10 +316,6 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
     for (int n = 0; n < C::NPV; ++n) acc[rg][n] = float4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  const rsrc_t kc = make_rsrc(a.k_cache, a.kc_bytes);
-  const rsrc_t vc = make_rsrc(a.v_cache, a.vc_bytes);
-  const rsrc_t ks = make_rsrc(a.k_scale, a.ks_bytes);
-  const rsrc_t vs = make_rsrc(a.v_scale, a.vs_bytes);
   // K8V3 codebook byte tables (fp16 of the fp32 codebook; the decode kernel's)
   uint32_t tlo03 = 0, tlo47 = 0, thi03 = 0, thi47 = 0;
   if constexpr (K8V3) {
@@ -368,70 +370,38 @@ __global__ __launch_bounds__(64 * kWavesOf<K8V3>, K8V3 ? 1 : 2) void verify_kern
         R.s = 1.0f;
         return;
       }
-      if constexpr (BIG) {  // one block holds the tile (block_size >= 32): descriptors rebased to its first row
-        const uint32_t r0 = __builtin_amdgcn_readfirstlane(row_of(base));
-        auto local = [&](int tt) -> uint32_t { return (uint32_t)(min(base + tt, u1 - 1) - base); };
-        const rsrc_t kt = window_rsrc(a.k_cache, a.kc_total, (uint64_t)r0 * D);
-        const rsrc_t vt = window_rsrc(a.v_cache, a.vc_total, (uint64_t)r0 * (K8V3 ? C::WORDS * 4 : D));
-        const rsrc_t kst = window_rsrc(a.k_scale, a.ks_total, (uint64_t)r0 * 4u);
-        const rsrc_t vst = window_rsrc(a.v_scale, a.vs_total, (uint64_t)r0 * (C::NB * 4u));
-#pragma unroll
-        for (int i = 0; i < C::LOADS; ++i) {
-          const int ch = tid + i * C::THREADS;
-          if (ch < C::CHUNKS) {
-            const int tt = ch / (D / 16), part = ch % (D / 16);
-            const uint32_t off = local(tt) * (uint32_t)D + (uint32_t)part * 16u;
-            R.k[i] = bload128(kt, off);
-            if constexpr (!K8V3) R.v[i] = bload128(vt, off);
-          }
-        }
-        if constexpr (K8V3) {
-          if (tid < C::VJOBS) {
-            const int grp = tid / C::SPLIT;
-            const int tt = grp / C::NG, gi = grp % C::NG;
-            const uint32_t off = local(tt) * (uint32_t)(C::WORDS * 4) + (uint32_t)gi * 12u;
-            const u32x3_t w = bload96(vt, off);
-            R.v[0].x = w.x;
-            R.v[0].y = w.y;
-            R.v[0].z = w.z;
-          }
-        }
-        if (tid < (1 + C::NB) * kTile) {
-          const uint32_t lr = local(tid & (kTile - 1));
-          const int nb = tid / kTile - 1;
-          R.s = __builtin_bit_cast(float, bload32(nb < 0 ? kst : vst, nb < 0 ? lr * 4u : (lr * C::NB + nb) * 4u));
-        }
-        return;
-      }
+      // one block holds the tile (block_size >= 32): descriptors rebased to its first row
+      const uint32_t r0 = __builtin_amdgcn_readfirstlane(row_of(base));
+      auto local = [&](int tt) -> uint32_t { return (uint32_t)(min(base + tt, u1 - 1) - base); };
+      const rsrc_t kt = window_rsrc(a.k_cache, a.kc_total, (uint64_t)r0 * D);
+      const rsrc_t vt = window_rsrc(a.v_cache, a.vc_total, (uint64_t)r0 * (K8V3 ? C::WORDS * 4 : D));
+      const rsrc_t kst = window_rsrc(a.k_scale, a.ks_total, (uint64_t)r0 * 4u);
+      const rsrc_t vst = window_rsrc(a.v_scale, a.vs_total, (uint64_t)r0 * (C::NB * 4u));
 #pragma unroll
       for (int i = 0; i < C::LOADS; ++i) {
         const int ch = tid + i * C::THREADS;
         if (ch < C::CHUNKS) {
           const int tt = ch / (D / 16), part = ch % (D / 16);
-          const uint32_t row = row_of(base + tt);
-          R.k[i] = bload128(kc, row * (uint32_t)D + (uint32_t)part * 16u);
-          if constexpr (!K8V3) R.v[i] = bload128(vc, row * (uint32_t)D + (uint32_t)part * 16u);
+          const uint32_t off = local(tt) * (uint32_t)D + (uint32_t)part * 16u;
+          R.k[i] = bload128(kt, off);
+          if constexpr (!K8V3) R.v[i] = bload128(vt, off);
         }
       }
       if constexpr (K8V3) {
         if (tid < C::VJOBS) {
           const int grp = tid / C::SPLIT;
           const int tt = grp / C::NG, gi = grp % C::NG;
-          const uint32_t off = row_of(base + tt) * (uint32_t)(C::WORDS * 4) + (uint32_t)gi * 12u;
-          const u32x3_t w = bload96(vc, off);
+          const uint32_t off = local(tt) * (uint32_t)(C::WORDS * 4) + (uint32_t)gi * 12u;
+          const u32x3_t w = bload96(vt, off);
           R.v[0].x = w.x;
           R.v[0].y = w.y;
           R.v[0].z = w.z;
         }
       }
-      if (tid < (1 + C::NB) * kTile) {  // k_scale of key tid, then block (tid/32 - 1)'s V scale
-        const uint32_t row = row_of(base + (tid & (kTile - 1)));
-        if constexpr (C::NB == 1) {
-          R.s = __builtin_bit_cast(float, bload32(tid < kTile ? ks : vs, row * 4u));
-        } else {
-          const int nb = tid / kTile - 1;
-          R.s = __builtin_bit_cast(float, bload32(nb < 0 ? ks : vs, nb < 0 ? row * 4u : (row * C::NB + nb) * 4u));
-        }
+      if (tid < (1 + C::NB) * kTile) {
+        const uint32_t lr = local(tid & (kTile - 1));
+        const int nb = tid / kTile - 1;
+        R.s = __builtin_bit_cast(float, bload32(nb < 0 ? kst : vst, nb < 0 ? lr * 4u : (lr * C::NB + nb) * 4u));
       }
     };
     // Window verify with fresh drafts: whether the tile at `base` holds
@@ -1783,16 +1753,19 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
   }
 }
 
-// The wide kernel serves the paged calls whose tensors
-// fit 32-bit offsets (no per-tile descriptor rebasing), with or without a
-// window.  Head_dim 256 in the 16-row kernel: its accumulators and q hi + lo
-// left no registers at two waves per SIMD (over 400 bytes of spills a lane);
-// one sequence of 1,999 queries over 6,007 keys, 4 KV heads, group 4: 2,200
-// -> 809 us; 7 dense prompts of up to 2,248, 8 heads over 4: 992 -> 244.
+// The wide kernel serves the paged calls whose tensors fit 32-bit offsets (no
+// per-tile descriptor rebasing), with or without a window.  Head_dim 256 in
+// the 16-row kernel: its accumulators and q hi + lo left no registers at two
+// waves per SIMD (408 to 484 bytes of scratch a lane); one sequence of 1,999
+// queries over 6,007 keys, 4 KV heads, group 4: 2,200 -> 809 us; 7 dense
+// prompts of up to 2,248, 8 heads over 4: 992 -> 244.  Some of the wide
+// kernel's paged instantiations spill too, to less scratch (bytes a lane, int8
+// / K8V3): head_dim 256 4-wave 68 / 104 (fresh drafts 148 / 180), narrow 256 /
+// 240; head_dim 128 8-wave 0 / 16 (fresh drafts 32 / 48), narrow 0 / 12;
+// head_dim 64, held to three workgroups a CU, 12 to 20 (fresh drafts 56).
 // Query rows per workgroup at this head_dim and layout (Cfg<D, K8V3>::ROWS,
 // or WideCfg::ROWS for the wide kernel), and the workgroups a CU keeps
 // resident (the kernels' launch bounds).
-static bool use_wide(bool big) { return !big; }
 // rows: query rows per (sequence, KV head) -- group x max_queries; the wide
 // kernel takes 8-wave workgroups at head_dim 128 when they exceed one 4-wave block
 static bool wide_eight(int head_dim, int rows) { return head_dim == 128 && rows > WideCfg<128, false, false>::ROWS; }
@@ -1916,13 +1889,13 @@ static int launch_combine(VerifyArgs& a, int64_t units, hipStream_t stream) {
   return check_launch("s8kv_verify_combine");
 }
 
-template <int D, bool K8V3, bool WIN, bool DENSE, bool BIG>
-static int launch_impl(VerifyArgs& a, hipStream_t stream) {
+template <int D, bool K8V3, bool WIN = false, bool DENSE = false>
+static int launch(VerifyArgs& a, hipStream_t stream) {
   static_assert(Cfg<D, K8V3>::ROWS == 16 * kWavesOf<K8V3> * (D <= 64 ? 2 : 1), "rows_per_wg");
   using C = Cfg<D, K8V3>;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_kernel<D, K8V3, WIN, DENSE, BIG>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&verify_kernel<D, K8V3, WIN, DENSE>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, WIN ? C::SMEM_WIN : C::SMEM) != hipSuccess) {
       set_error("s8kv_verify: cannot set the dynamic LDS size");
       return S8KV_ERR_LAUNCH;
@@ -1935,7 +1908,7 @@ static int launch_impl(VerifyArgs& a, hipStream_t stream) {
     set_error("s8kv_verify: grid too large");
     return S8KV_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((verify_kernel<D, K8V3, WIN, DENSE, BIG>), dim3((unsigned)grid), dim3(C::THREADS),
+  hipLaunchKernelGGL((verify_kernel<D, K8V3, WIN, DENSE>), dim3((unsigned)grid), dim3(C::THREADS),
                      WIN ? C::SMEM_WIN : C::SMEM, stream, a);
   if (a.splits > 1) {
     const int rc = check_launch("s8kv_verify");
@@ -1943,13 +1916,6 @@ static int launch_impl(VerifyArgs& a, hipStream_t stream) {
     return launch_combine<D, C::ROWS>(a, (int64_t)P * a.n_qblocks, stream);
   }
   return check_launch("s8kv_verify");
-}
-template <int D, bool K8V3, bool WIN = false, bool DENSE = false>
-static int launch(VerifyArgs& a, hipStream_t stream) {
-  if constexpr (DENSE)
-    return launch_impl<D, K8V3, WIN, DENSE, false>(a, stream);
-  else  // (the wide kernel serves the others)
-    return launch_impl<D, K8V3, WIN, DENSE, true>(a, stream);
 }
 
 template <int D, bool K8V3, bool DENSE, bool WIN, bool FRESH, bool EIGHT, bool NARROW>
@@ -2181,7 +2147,7 @@ static int verify_setup(verify::VerifyArgs& a, const void* q, int batch, int num
   a.k_scale = k_scale;
   a.kc_total = (uint64_t)(rows * head_dim);
   a.ks_total = (uint64_t)(rows * 4);
-  a.kc_bytes = cap_u32(a.kc_total);  // (BIG: unused by the tiles)
+  a.kc_bytes = cap_u32(a.kc_total);  // (past 4 GiB: unused by the tiles)
   a.ks_bytes = cap_u32(a.ks_total);
   a.block_table = block_table;
   a.bt_stride = block_table_stride;
@@ -2190,7 +2156,7 @@ static int verify_setup(verify::VerifyArgs& a, const void* q, int batch, int num
   a.tree_mask = tree_mask;
   a.bs_log2 = log2i(block_size);
   a.max_context_len = max_context_len;
-  const int rows_wg = verify::rows_per_wg(head_dim, k8v3, verify::use_wide(a.big), a.group * max_queries);
+  const int rows_wg = verify::rows_per_wg(head_dim, k8v3, !a.big, a.group * max_queries);
   a.n_qblocks = (a.group * max_queries + rows_wg - 1) / rows_wg;
   a.qscale = (float)((double)scale * 1.4426950408889634 / __builtin_sqrt((double)head_dim));
   a.out = (_Float16*)out;
@@ -2215,7 +2181,7 @@ static int verify_int8_impl(const void* q, int batch, int num_q_heads, int num_k
                               prefix_lens, query_lens, tree_mask, max_context_len, scale, out, false);
   if (rc != S8KV_OK) return rc;
   a.window = window;
-  const bool wide = verify::use_wide(a.big);
+  const bool wide = !a.big;
   if (const int rc = verify_use_workspace(a, head_dim, false, wide, workspace, workspace_bytes)) return rc;
   if (fresh_k) {
     S8KV_REQUIRE(fresh->v != nullptr && window > 0, S8KV_ERR_INVALID, "verify: fresh drafts need V and a window");
@@ -2313,7 +2279,7 @@ static int verify_k8v3_impl(const void* q, int batch, int num_q_heads, int num_k
                               prefix_lens, query_lens, tree_mask, max_context_len, scale, out, true);
   if (rc != S8KV_OK) return rc;
   a.window = window;
-  const bool wide = verify::use_wide(a.big);
+  const bool wide = !a.big;
   if (const int rc = verify_use_workspace(a, head_dim, true, wide, workspace, workspace_bytes)) return rc;
   if (fresh_k) {
     S8KV_REQUIRE(fresh->v != nullptr && window > 0, S8KV_ERR_INVALID, "verify: fresh drafts need V and a window");
