@@ -306,14 +306,17 @@ int s8kv_decode_window_k8v3(const void* q, int batch, int num_q_heads, int num_k
  * s >= query_lens[b] produce zeros.  head_dim 64, 128 or 256.
  *
  * workspace (16-byte aligned, s8kv_verify_workspace_size bytes) lets a call
- * with fewer (sequence, KV head, query block) units than the GPU keeps
- * resident split each unit's keys across workgroups and combine their
- * partials in a second kernel on the same stream (NULL or smaller: no split,
- * a slower call); a call whose units read more than 2^20 keys must split
+ * split the keys of its (sequence, KV head, query block) units across
+ * workgroups and combine their partials in a second kernel on the same stream
+ * (NULL or smaller: no split, a slower call).  A split is planned where the
+ * units are fewer than the GPU keeps resident, where a batch of more than one
+ * row has long rows (which would run alone at the end) and where a head has at
+ * most 32 query rows; a call whose units read more than 2^20 keys must split
  * (that bounds the rounding of one workgroup's fp32 sums), and without the
  * workspace it fails with S8KV_ERR_WORKSPACE.  Calls that overlap on one
- * workspace race.  The size covers both layouts (s8kv_verify_int8 and
- * s8kv_verify_k8v3 group query rows differently).
+ * workspace race.  The size covers both layouts and pools of any size, whose
+ * kernels group query rows differently (0: no split; at most about 0.56 GB on
+ * 256 CUs up to 2^20 keys, usually tens of MB).
  */
 int64_t s8kv_verify_workspace_size(int batch, int num_q_heads, int num_kv_heads, int head_dim, int max_queries,
                                    int max_context_len);

@@ -1776,8 +1776,13 @@ static bool wide_eight(int head_dim, int rows) { return head_dim == 128 && rows 
 static bool dense_eight(int pairs, int head_dim, int rows) {
   return wide_eight(head_dim, rows) && (int64_t)pairs * ((rows + 255) / 256) >= device_cus();
 }
-// ... and narrow ones when they fit one wave (one block either way, so only the
-// launch cares that dense calls and fresh drafts keep the 4-wave ones)
+// ... and narrow ones when they fit one wave.  Dense calls and fresh drafts of so
+// few rows keep the 4-wave ones (one block either way).  Fresh drafts are split
+// by the narrow workgroups' rule all the same, us a call unsplit / planned / in
+// the best of 1 to 32 splits: 5 queries, window 4,096, 8 heads, head_dim 128,
+// batch 1 173 / 23.0 / 23.8, ragged batch 32 182 / 120 / 115 (K8V3, 8 queries
+// 194 / 128 / 122); head_dim 256, 4 heads, window 1,024, batch 16 118 / 53 / 54;
+// head_dim 64, 16 heads, window 4,096, batch 32 157 / 125 / 119.
 static bool wide_narrow(int rows) { return rows <= WideCfg<128, false, false, true>::ROWS; }
 static int rows_per_wg(int head_dim, bool k8v3, bool wide, int rows) {
   if (wide)

@@ -169,9 +169,49 @@ def test_block_id_past_the_pool_reads_zeros(kind, d, nq, bs):
     assert np.isfinite(outs[0]).all() and np.array_equal(*outs)
 
 
+@pytest.mark.parametrize("kind,d", [("int8", 64), ("int8", 128), ("k8v3", 128), ("int8", 256), ("k8v3", 256)])
+@pytest.mark.parametrize("nq", [5, 20, 50])  # of 4 heads: one 32-row wave, a 128-row workgroup, more
+@pytest.mark.parametrize("given", ["none", "short"])
+def test_call_without_its_workspace_runs_unsplit(kind, d, nq, given, monkeypatch):
+    """No workspace, or one too small for any split: the bits of the unsplit
+    call; and beyond 2^20 keys, where a split is a must, an error."""
+    lib, inputs, asked = _lib.load(), ops._verify_inputs, []
+
+    def withheld(*args, **kw):
+        keep, head, tail, (ptr, size), geo, out = inputs(*args, **kw)
+        asked.append(size)
+        return keep, head, tail, (None, 0) if given == "none" else (ptr, min(size, 4096)), geo, out
+
+    def run(max_ctx=None):
+        out = fn(q, *cache, *extra, table, prefix, 64, max_context_len=max_ctx or int(case.lens.max()),
+                 scale=case.scale)
+        torch.cuda.synchronize()
+        return out
+
+    lens = np.array([9000, 33, 4100])
+    case = make_case(98 + d, 3, 8, 2, d, 64, lens + nq, width=(1 << 20) // 64 + 1)
+    cache = alloc(kind, case.num_blocks, 2, 64, d)
+    append(kind, t(case.k), t(case.v), cache, t(case.slots))
+    q = t(np.random.default_rng(99).standard_normal((3, 8, nq, d)).astype(np.float16))
+    table, prefix = t(case.block_table), t(lens.astype(np.int32))
+    fn = ops.attn_paged_verify if kind == "int8" else ops.attn_paged_verify_k8v3
+    extra = () if kind == "int8" else (t(CODEBOOK),)
+    split = run()
+    lib.s8kv_verify_set_splits(1)
+    try:
+        whole = run()
+    finally:
+        lib.s8kv_verify_set_splits(0)
+    monkeypatch.setattr(ops, "_verify_inputs", withheld)
+    got = run()
+    assert asked[0] > 0 and torch.equal(got, whole) and not torch.equal(split, whole)
+    assert_close(to_np(got.float()), to_np(split.float()).astype(np.float64), f"{kind} D={d} unsplit")
+    with pytest.raises(RuntimeError, match="workspace"):
+        run((1 << 20) + 1)
+
+
 def test_workspace_counts_the_split():
-    """The workspace query plans the ragged batch's split too, and a call
-    without a workspace runs unsplit."""
+    """The workspace query plans the ragged batch's split too."""
     lib = _lib.load()
     assert lib.s8kv_verify_workspace_size(32, 32, 8, 128, 5, 8192) > 0
     assert lib.s8kv_verify_workspace_size(32, 32, 8, 128, 5, 500) == 0
