@@ -1437,10 +1437,11 @@ __launch_bounds__((WideCfg<D, K8V3, EIGHT>::THREADS), (WideCfg<D, K8V3, EIGHT>::
       // round, a barrier between the halves.  In step, as one barrier a tile
       // leaves them, both used the matrix cores and then the VALU at the same
       // time.  With the scalar addresses below, us a call, before -> now:
-      // 16 x 512-query chunk over 4,096 keys 1,077 -> 1,024 (8 % fewer cycles, but the
+      // 16 x 512-query chunk over 4,096 keys 1,142 -> 1,091 (8 % fewer cycles, but the
       // matrix cores then run the clock down: 2.13 -> 2.0 GHz; without any
-      // softmax or staging it would be 790, at 1.73 GHz); 32 trees of 16 to
-      // 64 nodes over 8,192 keys 448 -> 413; 12 ragged dense prompts 854 -> 751.
+      // softmax or staging 790 where the whole took 1,024, at 1.73 GHz); 32 trees
+      // of 16 to 64 nodes over 8,192 keys 466 -> 439; 12 ragged dense prompts
+      // 920 -> 821.
       //   half 2t    : waves 0-3  PV(t-1), QK(t)          waves 4-7  softmax(t-1), V(t) -> LDS
       //   half 2t + 1: waves 0-3  softmax(t), K(t+1) -> LDS   waves 4-7  PV(t-1), QK(t)
       // K(t+1) replaces K(t-1), last read in half 2t - 1, and V(t) replaces
